@@ -16,9 +16,10 @@
 // dequantise-then-fp32, accumulated in fp32.
 //
 // Fragment order: an MFMA lane holds 8 inputs in the order 0 4 1 5 2 6 3 7 of an 8-input
-// chunk, the order in which the nibble masking (w >> 4 j) & 0x000f000f (and the int8 / fp8
-// byte pairing) produces bf16 pairs; token tiles in LDS are stored in the same permuted
-// order, 16-byte chunk b of token t at b ^ (t % 16), so the 16 token rows of one read spread
+// chunk, the order in which the nibble masking (w >> 4 j) & 0x000f000f (and the int8 byte
+// pairing) produces bf16 pairs, or in input order for fp8 (v_cvt_scalef32_pk_bf16_fp8 converts
+// neighbouring bytes: one instruction per two weights); token tiles in LDS are stored in the
+// same order, 16-byte chunk b of token t at b ^ (t % 16), so the 16 token rows of one read spread
 // over all banks and each A fragment is one 16-byte LDS read.  The per-kernel comments give
 // the lane -> input mapping of each weight format.
 #include <mutex>
@@ -33,13 +34,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int PF_WPB = 8;     // waves per block (k_grouped_ks)
-constexpr int PF_GWPB = 8;    // waves per block (k_grouped)
+constexpr int PF_GWPB = 8;    // waves per block (k_grouped, k_grouped_pass)
 // 16-row tiles per wave and item (k_grouped).  Measured: 2 (one token tile serving both) is
 // level with 1 at 300 prefill rows and 20% slower at 4 decode rows (fewer, larger items)
 constexpr int PF_GRPW = 1;
-constexpr int PF_TOK = 16;    // tokens per pass (one MFMA tile)
-constexpr int PF_MAXE = 256;  // experts
+constexpr int PF_TOK = 16;    // tokens of one MFMA tile (and of a pass of k_grouped)
 constexpr int PF_DEPTH = 4;   // 4-group weight steps in flight per wave (k_grouped)
+constexpr int PF_MAXE = 256;  // experts
 
 DEV f32x4 mfma(const uint4& a, const uint4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
@@ -59,11 +60,6 @@ struct FmtQ4 {
   static DEV size_t row_bytes(int K) { return (size_t)K / 2; }
   // fragment bytes of (row, group G) for lane group g: 8 bytes = 16 nibbles
   static DEV void load(const uint8_t* row, int G, int g, uint2& raw) { raw = ld8(row + G * 32 + g * 8); }
-  static DEV void convert(const uint2& raw, uint4& a0, uint4& a1) {
-    const uint32_t m = 0x000f000fu, b = 0x43004300u;
-    a0 = make_uint4((raw.x & m) | b, ((raw.x >> 4) & m) | b, ((raw.x >> 8) & m) | b, ((raw.x >> 12) & m) | b);
-    a1 = make_uint4((raw.y & m) | b, ((raw.y >> 4) & m) | b, ((raw.y >> 8) & m) | b, ((raw.y >> 12) & m) | b);
-  }
   // (scale, min) of row n, group G: raw word, then decoded
   static DEV uint32_t scale_raw(const void* S, size_t n, int G, int K) {
     return reinterpret_cast<const uint32_t*>(S)[n * (K / 64) + G];
@@ -72,8 +68,7 @@ struct FmtQ4 {
   static DEV float2 scale(const void* S, size_t n, int G, int K) { return scale_val(scale_raw(S, n, G, K)); }
 };
 
-// element order inside an 8-element fragment: perm = 0 4 1 5 2 6 3 7
-// int8: 16 bytes per lane and group; bytes k..k+15 of the group slice, reordered
+// int8 (fragments in the order 0 4 1 5 2 6 3 7): 16 bytes per lane and group; bytes k..k+15 of the group slice, reordered
 template <class SH>
 struct FmtQ8 {
   using Scale = SH;
@@ -113,18 +108,14 @@ struct FmtFP8 {
   static constexpr int scale_group = 128;
   static DEV size_t row_bytes(int K) { return (size_t)K; }
   static DEV void load(const uint8_t* row, int G, int g, uint4& raw) { raw = ld16(row + G * 64 + g * 16); }
-  static DEV uint32_t pk(float a, float b) { return (__float_as_uint(b) & 0xffff0000u) | (__float_as_uint(a) >> 16); }
-  // e4m3 -> f32 is exact, and every e4m3 value is a bf16 value
-  static DEV uint4 frag(uint32_t lo, uint32_t hi) {
-    const float l0 = __builtin_amdgcn_cvt_f32_fp8(lo, 0), l1 = __builtin_amdgcn_cvt_f32_fp8(lo, 1);
-    const float l2 = __builtin_amdgcn_cvt_f32_fp8(lo, 2), l3 = __builtin_amdgcn_cvt_f32_fp8(lo, 3);
-    const float h0 = __builtin_amdgcn_cvt_f32_fp8(hi, 0), h1 = __builtin_amdgcn_cvt_f32_fp8(hi, 1);
-    const float h2 = __builtin_amdgcn_cvt_f32_fp8(hi, 2), h3 = __builtin_amdgcn_cvt_f32_fp8(hi, 3);
-    return make_uint4(pk(l0, h0), pk(l1, h1), pk(l2, h2), pk(l3, h3));
+  // 16 e4m3 bytes -> two bf16 fragments in input order (exact: every e4m3 value is a bf16 value)
+  static DEV void frags(const uint4& raw, uint4& a0, uint4& a1) {
+    a0 = make_uint4(cvt2<false>(raw.x), cvt2<true>(raw.x), cvt2<false>(raw.y), cvt2<true>(raw.y));
+    a1 = make_uint4(cvt2<false>(raw.z), cvt2<true>(raw.z), cvt2<false>(raw.w), cvt2<true>(raw.w));
   }
-  static DEV void convert(const uint4& raw, uint4& a0, uint4& a1) {
-    a0 = frag(raw.x, raw.y);
-    a1 = frag(raw.z, raw.w);
+  template <bool HI>
+  static DEV uint32_t cvt2(uint32_t w) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
   }
   // scale of row n, 64-group G: block (n / 128, G / 2); S points at this expert's blocks
   static DEV uint32_t scale_raw(const void* S, size_t n, int G, int K) {
@@ -150,6 +141,8 @@ struct Raw<FmtFP8<SF>> {
   using T = uint4;
 };
 
+// ---- grouped experts ---------------------------------------------------------------------------
+
 // Spin until an LDS counter reaches target (acquire); bounded, so a broken protocol ends the
 // wait instead of hanging the GPU, and then raises DR_ERR_PREFILL_WAIT in the library error
 // word (the results of the launch are wrong; dr_stream_sync and dr_last_error report it).
@@ -165,7 +158,7 @@ DEV void lds_count(uint32_t* c) {
 }
 
 // Token tile of tokens [row0, row0 + ntok) x all K inputs of a bf16 row matrix, staged into LDS
-// in the permuted fragment order: 16-byte block r of token t at t * K / 8 + (r ^ t), the xor
+// in the fragment order of the weights (int4: permuted): 16-byte block r of token t at t * K / 8 + (r ^ t), the xor
 // spreading the 16 tokens of one read over distinct LDS banks; rows beyond ntok are zero.
 // Split in two so the caller can issue its first weight loads between the token loads and
 // the LDS stores: the stores wait only for the token loads issued before those weight loads.
@@ -226,8 +219,9 @@ struct TokTile {
         const int r = b % (K / 8);
         if ((r & 7) == 0) reinterpret_cast<float*>(xs + PF_TOK * K / 8)[16 * (r >> 3) + t] = sum;
       }
-      // (e0 e1)(e2 e3)(e4 e5)(e6 e7) -> (e0 e4)(e1 e5)(e2 e6)(e3 e7)
+      // int4: (e0 e1)(e2 e3)(e4 e5)(e6 e7) -> (e0 e4)(e1 e5)(e2 e6)(e3 e7)
       xs[b ^ (t & 15)] =
+          !with_sums ? v[i] :
           make_uint4(__builtin_amdgcn_perm(v[i].z, v[i].x, 0x05040100u), __builtin_amdgcn_perm(v[i].z, v[i].x, 0x07060302u),
                      __builtin_amdgcn_perm(v[i].w, v[i].y, 0x05040100u), __builtin_amdgcn_perm(v[i].w, v[i].y, 0x07060302u));
     }
@@ -241,18 +235,18 @@ struct TokTile {
 // (one 64-byte run per row per load: half the cache-line requests of 8-byte loads); all four
 // (scale, min) words of the step come in one 16-byte load.
 template <class F, bool P = F::paired>
-struct Step {
+struct Step4 {
   typename Raw<F>::T raw[4];
   uint32_t sc[4];
 };
 template <class F>
-struct Step<F, true> {
+struct Step4<F, true> {
   uint4 raw[2];
   uint4 sc;
 };
 
 template <class F>
-DEV void load_step(const uint8_t* row, const void* ws, size_t n, int G0, int g, int K, Step<F>& s) {
+DEV void load_step4(const uint8_t* row, const void* ws, size_t n, int G0, int g, int K, Step4<F>& s) {
   if constexpr (F::paired) {
     s.raw[0] = ld16(row + G0 * 32 + g * 16);
     s.raw[1] = ld16(row + G0 * 32 + 64 + g * 16);
@@ -260,20 +254,45 @@ DEV void load_step(const uint8_t* row, const void* ws, size_t n, int G0, int g, 
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) F::load(row, G0 + i, g, s.raw[i]);
-    if (F::scale_group != 0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s.sc[i] = F::scale_raw(ws, n, G0 + i, K);
-    }
+    for (int i = 0; i < 4; ++i) s.sc[i] = F::scale_raw(ws, n, G0 + i, K);
   }
 }
 
+// k_grouped_pass: weights of one step (a 16-row tile x STEP inputs, 2 KB) per lane.  int4, 256 inputs: the four
+// lanes of a row read the 64 bytes of groups (G0 + 2 p, G0 + 2 p + 1) as 16 bytes each, raw[p] =
+// bytes 16 g of that span (lanes g = 0, 1 hold the first group, g = 2, 3 the second), and the
+// row's four (scale, min) words.  fp8, 128 inputs: raw[i] = bytes 16 g of group G0 + i, and the
+// block's scale.
+template <class F, bool P = F::paired>
+struct Step {
+  uint4 raw[2];
+  uint32_t sc;
+};
+template <class F>
+struct Step<F, true> {
+  uint4 raw[2];
+  uint4 sc;
+};
+
+// the kernel's lambdas are inlined before any other optimisation: arrays they capture then live in
+// registers
+#define PF_INL __attribute__((always_inline))
+
+// c ? a : b by value (a conditional lvalue would keep the operands in memory)
+template <class T>
+DEV T pick(bool c, T a, T b) {
+  return c ? a : b;
+}
+
 // nibbles of one 32-bit word -> bf16 fragment 128 + q in the order 0 4 1 5 2 6 3 7 with
-// m = 0x000f000f, b = 0x43004300; m = b = 0 gives the zero fragment (a lane left out)
+// m = 0x000f000f, b = 0x43004300
 DEV uint4 q4_frag(uint32_t w, uint32_t m, uint32_t b) {
   return make_uint4((w & m) | b, ((w >> 4) & m) | b, ((w >> 8) & m) | b, ((w >> 12) & m) | b);
 }
 
-// MODE 0: gate_up (row pairs j, I + j; writes bf16 silu(g) u)   MODE 1: down (writes f32)
+// Experts of few tokens (use_passes).  MODE 0: gate_up (row pairs j, I + j; writes bf16 silu(g) u)
+// MODE 1: down (writes f32)
 //
 // Work items: (expert e, 16-token pass p < ceil(counts[e] / 16), row block yb).  A persistent
 // grid of resident blocks walks them (item = blockIdx.x, + gridDim.x, ...).  Each wave owns one
@@ -285,11 +304,11 @@ DEV uint4 q4_frag(uint32_t w, uint32_t m, uint32_t b) {
 // tokens just before them), and the tokens are stored into the second of two LDS tile buffers
 // at the boundary, so one barrier per item is the only gap.  MFMA operands: A = tokens (lane: token l % 16),
 // B = weights (lane: row l % 16), so D[token 4 (l / 16) + i][row l % 16] sits in lane l: one
-// weight row per lane, one (scale, min) pair per group.  The group input sums X_g come from an
-// MFMA against bf16 ones (int4: staged with the tokens).
-// PK (int4 only): the weights are in the tile-step layout of dr_moe_pack_q4, so each step of a
-// wave is one contiguous 2048-byte block (two 1024-byte wave loads) and 256 bytes of scales,
-// where the reference layout gives 16 rows x 128 bytes 1 KB apart.
+// weight row per lane, one (scale, min) pair per group.  The group input sums X_g (int4)
+// are staged with the tokens.
+// PK: the weights are in the tile-step layout of dr_moe_pack_q4 / dr_moe_pack_fp8, so each step of a
+// wave is one contiguous block (int4: two 1024-byte wave loads and 256 bytes of scales) where the
+// reference layout gives 16 rows x 128 bytes 1 KB apart.
 template <class F, int MODE, int K, bool GATHER, bool PK = false>
 __global__ void __launch_bounds__(PF_GWPB * 64)
     k_grouped(const uint8_t* __restrict__ Wq, const void* __restrict__ Ws, const uint16_t* __restrict__ X,
@@ -400,7 +419,7 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
   auto row_of = [&](const Item& it, int t) {
     return (size_t)(up ? N / 2 : 0) + (size_t)(((it.yb * PF_GRPW + t) * WR + wt) * 16 + c16);
   };
-  auto fetch = [&](const Item& it, int s, Step<F>& st) {
+  auto fetch = [&](const Item& it, int s, Step4<F>& st) {
     const size_t n = row_of(it, s / SPT);
     if constexpr (PK && F::paired) {
       // int4 block (tile n / 16, step): lane l's 16 bytes of each half are what load_step reads
@@ -421,10 +440,9 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
 #pragma unroll
       for (int i = 0; i < 4; ++i) st.sc[i] = F::scale_raw(it.ws, n, G0 + i, K);
     } else {
-      load_step<F>(it.wq + n * rb, it.ws, n, (s % SPT) * 4, g, K, st);
+      load_step4<F>(it.wq + n * rb, it.ws, n, (s % SPT) * 4, g, K, st);
     }
   };
-  const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
   // the int4 conversion constants live in VGPRs: v_and_or_b32 (VOP3) takes no literal
   // operands on this architecture and at most one scalar one, so with literals the
   // conversion would cost two instructions per dword instead of one
@@ -434,7 +452,7 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
   Item cur = item_at(blockIdx.x);
   if (!cur.valid) return;
   Item nxt = item_at(blockIdx.x + gridDim.x);
-  Step<F> ring[DEPTH];  // steps in flight
+  Step4<F> ring[DEPTH];  // steps in flight
   TokTile<K, PF_GWPB * 64> tt;
   // Waves synchronise per item through LDS counters instead of a block barrier, so they may
   // drift by up to half an item: n_stored = 8 (k + 1) once every wave stored its part of item
@@ -495,7 +513,7 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
     const uint4* xu8 = xrow + ((8 + 2 * g) ^ c16);
     const uint4* xu9 = xrow + ((9 + 2 * g) ^ c16);
     f32x4 tA = {0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const Step<F>& sa, int G0) {
+    auto compute = [&](const Step4<F>& sa, int G0) {
       if constexpr (F::paired) {
         // min term of the step's four groups as one fp32 MFMA: A = group sums X[token c16][G0 + g],
         // B = (m - 128 s)[row c16][G0 + g] (this lane's scale word g)
@@ -544,21 +562,11 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
           const uint4 x0 = (G & 1 ? xu8 : xu0)[16 * (G >> 1)], x1 = (G & 1 ? xu9 : xu1)[16 * (G >> 1)];
           const f32x4 z = {0.f, 0.f, 0.f, 0.f};
           uint4 a0, a1;
-          F::convert(sa.raw[i], a0, a1);
-          if (F::scale_group == 0) {
-            tA = mfma(x1, a1, mfma(x0, a0, tA));
-          } else {
-            const f32x4 accA = mfma(x1, a1, mfma(x0, a0, z));
-            f32x4 xg = z;
-            if (F::has_min) xg = mfma(x1, ones, mfma(x0, ones, z));
-            const float2 pa = F::scale_val(sa.sc[i]);
-            const float ca = pa.y - 128.f * pa.x;
+          F::frags(sa.raw[i], a0, a1);
+          const f32x4 accA = mfma(x1, a1, mfma(x0, a0, z));
+          const float pa = F::scale_val(sa.sc[i]).x;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              tA[r] = __builtin_fmaf(pa.x, accA[r], tA[r]);
-              if (F::has_min) tA[r] = __builtin_fmaf(ca, xg[r], tA[r]);
-            }
-          }
+          for (int r = 0; r < 4; ++r) tA[r] = __builtin_fmaf(pa, accA[r], tA[r]);
         }
       }
       // the sums are materialised here, each step: otherwise the compiler sinks the scale
@@ -595,9 +603,6 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
       // gate waves keep g until the boundary
       const int t = i / SPT;
       const size_t n = row_of(cur, t);
-      const float rs = F::scale_group == 0 ? F::scale(cur.ws, n, 0, K).x : 1.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) tA[r] *= rs;
       if (MODE == 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -627,6 +632,458 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
   if (MODE == 0 && !up && pend.valid) finish_gate(pend, k);  // the last item
   // no wave may leave while others still count on its LDS (the counters live in it)
   lds_barrier();
+}
+
+// Experts of more tokens (use_passes).  MODE 0: gate_up (row pairs j, I + j; writes bf16 silu(g) u)
+// MODE 1: down (writes f32)
+//
+// Work items: (expert e, pass of up to PASS tokens, row block).  A persistent grid of resident
+// blocks walks them (item = blockIdx.x, + gridDim.x, ...).  A wave owns two 16-row tiles of an item
+// (gate_up: a gate tile and the matching up tile; down: two neighbouring tiles) against the
+// pass's token tiles of 16, so a weight fragment is dequantised once for the whole pass and a
+// token fragment read from LDS once for both tiles (k_grouped does both per 16 tokens and tile).
+// The whole item sequence of a block is one stream of steps (STEP inputs of every tile): step s
+// computes from the weight ring and token slice s in LDS, then stores slice s + 1 to LDS
+// (registers -> LDS, double buffered; one barrier per step), requests slice s + 3 and the weights of
+// step s + 4 into the slot just used.  The order of those requests keeps two to three steps of weights in
+// flight (110 KB per CU): loads return in order, and the wait for slice s + 1 leaves everything
+// requested after it outstanding.
+// MFMA operands: A = tokens (lane: token l % 16), B = weights (lane: row l % 16), so
+// D[token 4 (l / 16) + i][row l % 16] sits in lane l: one weight row per lane, one (scale, min)
+// pair per group.  An output's sums depend neither on the pass or tile its token falls in nor on the
+// kernel (the same operations in the same order as k_grouped, so the same bits).
+// What bounds it: at one token tile per pass the steps run at the HBM rate (1.55 us for 36.8 KB per
+// CU, 6.1 TB/s); with two int4 tiles the dequantisation and MFMA issue of a step (1.9 us) do.
+// Measured (tile-step copy, gate_up / down, k_grouped -> k_grouped_pass): int4 1024 rows 143 / 78 -> 112 / 66 us,
+// fp8 600 rows with hot experts 124 / 68 -> 117 / 60 us; int4 300 rows 68 / 37.7 -> 67 / 41 us (use_passes).
+// Not kept: 16-row tiles with two blocks per CU (132 / 72 us at 1024 rows), passes of 48 and 64
+// int4 tokens (the ring, two slices and the sums exceed 256 registers: spills), rotating
+// the steps per expert, row-pair loads of whole cache lines in the reference layout (no change).
+// PK: the weights are in the tile-step layout of dr_moe_pack_q4 / dr_moe_pack_fp8, so a step of
+// a tile is one contiguous 2048-byte block where the reference layout gives 16 runs of 128 bytes.
+template <class F, int MODE, int K, bool GATHER, bool PK>
+__global__ void __launch_bounds__(PF_GWPB * 64)
+    k_grouped_pass(const uint8_t* __restrict__ Wq, const void* __restrict__ Ws, const uint16_t* __restrict__ X,
+              const int* __restrict__ offsets, const int* __restrict__ counts, void* __restrict__ out, int N,
+              size_t expert_q_bytes, size_t expert_s_elems, int s_elem_bytes, int E, const int* __restrict__ rmap,
+              int x_rows) {
+  constexpr int STEP = F::paired ? 256 : 128;      // inputs per step
+  constexpr int PASS = F::paired ? 32 : 64;        // tokens per pass (48 and 64 spill for int4)
+  constexpr int RT = 2;                            // 16-row tiles per wave
+  constexpr int SPT = K / STEP;                    // steps per item
+  constexpr int BR = STEP / 8;                     // 16-byte blocks of a token's slice
+  constexpr int NT = PF_GWPB * 64, TPL = NT / BR;  // threads; tokens per load round
+  constexpr int NL = PASS / TPL;                // load rounds per slice
+  constexpr int SLICE = PASS * BR + (F::paired ? PASS : 0);  // LDS blocks: the slice, its group sums
+  constexpr int DEPTH = 4;                         // weight steps in the ring
+  constexpr int NI = SPT % DEPTH == 0 ? 1 : 2;     // items per round of the ring
+  static_assert((NI * SPT) % DEPTH == 0 && SPT % 2 == 0, "ring slots and slice buffers must be static");
+  __shared__ uint4 slices[2 * SLICE];
+  __shared__ int ends[PF_MAXE];  // passes of experts 0 .. e
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int g = lane >> 4, c16 = lane & 15;
+  // inclusive prefix of the experts' pass counts, by every wave (the same values)
+  int n_pass;
+  {
+    int pl[4], psum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = counts[min(4 * lane + j, E - 1)];
+      pl[j] = 4 * lane + j < E ? (c + PASS - 1) / PASS : 0;
+      psum += pl[j];
+    }
+    int incl = psum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(incl, o);
+      if (lane >= o) incl += t;
+    }
+    n_pass = __builtin_amdgcn_readfirstlane(__shfl(incl, 63));  // wave-uniform, in a scalar register
+    int end = incl - psum;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) end += pl[j], ends[4 * lane + j] = end;
+  }
+  if (n_pass == 0) return;
+  lds_barrier();
+  const int G = gridDim.x;
+  constexpr int TROWS = MODE == 0 ? 16 : 32;  // output columns per wave
+  const int NO = MODE == 0 ? N / 2 : N;
+  // waves with rows of their own: all, or fewer (the others repeat them and store nothing) where
+  // the items would not fill the grid
+  int AW = PF_GWPB;
+  while (AW > 2 && n_pass * (NO / (TROWS * AW)) < G) AW >>= 1;
+  const int YB = NO / (TROWS * AW);  // row blocks per expert
+  const int n_items = n_pass * YB;
+  const int wt = wave & (AW - 1);
+  struct Item {
+    const uint8_t* wq;
+    const char* ws;
+    int row0;      // first token slot of the pass
+    int ntok, n0;  // tokens; first weight row of this wave's first tile
+    bool valid;
+  };
+  // Item i -> (flat pass q, row block yb).  Blocks run on XCD blockIdx % 8, each XCD with its
+  // own L2: where the grid allows, the YB row blocks of a pass go to blocks of one XCD in the
+  // same round of gridDim.x items, so its token rows are fetched into that L2 once, and
+  // consecutive passes to different XCDs, so a last partial round is spread over them (round r,
+  // block b = x + 8 j: q = 8 (r EPR + j / YB) + x, yb = j % YB with EPR passes per XCD and
+  // round).  Otherwise q = i % n_pass, yb = i / n_pass.  Indices past the last pass are
+  // invalid; they map to pass 0, row block 0 (loaded, never computed).
+  // Lane k of every wave works out item base + k of its block, 64 items at a time; an item is
+  // then two lane reads.
+  const int EPR = (G / 8) / YB;
+  const bool xcd_map = G % 8 == 0 && EPR > 0 && (G / 8) % YB == 0;
+  int li, lr;  // e | yb << 8 | ntok << 16 | valid << 24, row0
+  auto items_from = [&](int base) PF_INL {
+    const int rnd = base + lane, b = blockIdx.x, j = b >> 3, i = rnd * G + b;
+    int q = xcd_map ? (rnd * EPR + j / YB) * 8 + (b & 7) : i % n_pass;
+    int yb = xcd_map ? j % YB : i / n_pass;
+    const bool valid = xcd_map ? q < n_pass : i < n_items;
+    if (!valid) q = 0, yb = 0;
+    int e = 0;  // first expert with ends[e] > q
+#pragma unroll
+    for (int s = PF_MAXE / 2; s > 0; s >>= 1)
+      if (ends[e + s - 1] <= q) e += s;
+    const int cnt = counts[e];
+    const int pass = q - (ends[e] - (cnt + PASS - 1) / PASS);
+    lr = offsets[e] + pass * PASS;
+    li = e | yb << 8 | min(PASS, cnt - pass * PASS) << 16 | (valid ? 1 << 24 : 0);
+  };
+  auto item_at = [&](int k) PF_INL {
+    if ((k & 63) == 0 && k > 0) items_from(k);
+    const int w = __builtin_amdgcn_readlane(li, k & 63);
+    const int e = w & 255;
+    Item it;
+    it.wq = Wq + (size_t)e * expert_q_bytes;
+    it.ws = reinterpret_cast<const char*>(Ws) + (size_t)e * expert_s_elems * s_elem_bytes;
+    it.row0 = __builtin_amdgcn_readlane(lr, k & 63);
+    it.ntok = (w >> 16) & 255;
+    it.n0 = (((w >> 8) & 255) * AW + wt) * TROWS;
+    it.valid = w >> 24;
+    return it;
+  };
+  constexpr size_t rb = F::paired ? K / 2 : K;  // bytes of a weight row
+  struct Weights {
+    Step<F> t[RT];
+  };
+  auto fetch = [&](const Item& it, int s, Weights& w) PF_INL {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int n0 = it.n0 + (r == 0 ? 0 : MODE == 0 ? N / 2 : 16);  // first row of the tile
+      Step<F>& st = w.t[r];
+      if constexpr (PK) {
+        const size_t blk = (size_t)(n0 >> 4) * SPT + s;
+        st.raw[0] = ld16(it.wq + blk * 2048 + lane * 16);
+        st.raw[1] = ld16(it.wq + blk * 2048 + lane * 16 + 1024);
+        if constexpr (F::paired) st.sc = ld16(it.ws + blk * 256 + c16 * 16);
+      } else {
+        const uint8_t* tb = it.wq + (size_t)n0 * rb + s * 128;
+        st.raw[0] = ld16(tb + c16 * rb + g * 16);
+        st.raw[1] = ld16(tb + c16 * rb + g * 16 + 64);
+        if constexpr (F::paired)
+          st.sc = ld16(it.ws + ((size_t)n0 * (K / 64) + s * 4) * 4 + (size_t)c16 * (K / 64) * 4);
+      }
+      if constexpr (!F::paired) st.sc = F::scale_raw(it.ws, (size_t)n0, 2 * s, K);
+    }
+  };
+  // token slice s of an item: thread b holds block b % BR of tokens b / BR + TPL i.  Rows come
+  // through a buffer resource: those past ntok read zeros without a fetch.  With GATHER lane t of
+  // a wave holds token t's row (read from the slot -> row map an item ahead).
+  const int tb_t = threadIdx.x / BR, tb_r = threadIdx.x % BR;
+  auto rows_of = [&](const Item& it) PF_INL { return GATHER ? rmap[it.row0 + min(lane, it.ntok - 1)] : 0; };
+  uint32_t off[NL];  // byte offset of this thread's block of slice 0 of the item being requested
+  auto offsets_of = [&](const Item& it, int rows) PF_INL {
+    constexpr int TPW = 64 / BR;  // tokens of one wave and load round
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      if constexpr (GATHER) {
+        int row = __builtin_amdgcn_readlane(rows, i * TPL + wave * TPW);
+#pragma unroll
+        for (int q = 1; q < TPW; ++q) row = pick(lane / BR == q, __builtin_amdgcn_readlane(rows, i * TPL + wave * TPW + q), row);
+        off[i] = i * TPL + tb_t < it.ntok ? (uint32_t)((row * K + tb_r * 8) * 2) : 0x7ffffff0u;
+      } else {
+        off[i] = (uint32_t)(((i * TPL + tb_t) * K + tb_r * 8) * 2);
+      }
+    }
+  };
+  struct Tok {
+    uint4 v[NL];
+  };
+  auto load_tok = [&](const Item& it, int s, Tok& t) PF_INL {
+    const __amdgpu_buffer_rsrc_t rs = GATHER
+        ? __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X), 0, x_rows * K * 2, 0x00020000)
+        : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X + (size_t)it.row0 * K), 0, it.ntok * K * 2, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      t.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off[i] + s * STEP * 2, 0, 0));
+  };
+  // registers -> LDS: 16-byte block r of token t at t BR + (r ^ (t & 15)), the xor spreading the 16
+  // tokens of one read over distinct banks.  int4: in the permuted fragment order, and the fp32 sum
+  // of every 64-input group of every token (for the min term) at float PASS G + t behind the slice.
+  const auto lds = [&](uint32_t o) PF_INL { return reinterpret_cast<char*>(slices) + o; };
+  // per-lane LDS byte offsets (kept opaque, so the slice buffer, tile and phase of an access go into its
+  // immediate offset instead of an address register each)
+  uint32_t st_x = (tb_t * BR + (tb_r ^ (tb_t & 15))) * 16, st_s = PASS * BR * 16 + (PASS * (tb_r >> 3) + tb_t) * 4;
+  asm volatile("" : "+v"(st_x), "+v"(st_s));
+  auto store_tok = [&](const Tok& tk, int buf, int ntok) PF_INL {
+    static_assert(TPL % 16 == 0, "every round of a thread has the same token index modulo 16");
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      if (i * TPL >= ((ntok + 15) & ~15)) break;  // tiles no wave reads
+      const uint4 v = tk.v[i];
+      uint4* xs = reinterpret_cast<uint4*>(lds(st_x + (buf * SLICE + i * TPL * BR) * 16));
+      if constexpr (F::paired) {
+        // 8 blocks of a group sit in 8 consecutive lanes
+        float sum = 0.f;
+        const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += __uint_as_float(wv[k] << 16) + __uint_as_float(wv[k] & 0xffff0000u);
+        sum = xsum_step<4>(xsum_step<2>(xsum_step<1>(sum)));
+        if ((tb_r & 7) == 0) *reinterpret_cast<float*>(lds(st_s + buf * SLICE * 16 + i * TPL * 4)) = sum;
+        // (e0 e1)(e2 e3)(e4 e5)(e6 e7) -> (e0 e4)(e1 e5)(e2 e6)(e3 e7)
+        *xs = make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
+                         __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));
+      } else {
+        *xs = v;
+      }
+    }
+  };
+  // token fragments: int4 reads blocks tb, tb + 1 (group A) and tb + 8, tb + 9 (group B) of each half slice
+  // (below), fp8 blocks 2 g, 2 g + 1 and 2 g + 8, 2 g + 9
+  const int tb = F::paired ? 4 * (g & 1) + 2 * (g >> 1) : 2 * g;
+  uint32_t ld_x[4], ld_s = PASS * BR * 16 + (PASS * g + c16) * 4;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ld_x[j] = (c16 * BR + ((tb + (j & 1) + 4 * (j & 2)) ^ c16)) * 16;
+  asm volatile("" : "+v"(ld_x[0]), "+v"(ld_x[1]), "+v"(ld_x[2]), "+v"(ld_x[3]), "+v"(ld_s));
+  auto tok_frag = [&](int buf, int t, int p, int j) PF_INL {
+    return *reinterpret_cast<const uint4*>(lds(ld_x[j] + (buf * SLICE + 16 * (BR * t + p)) * 16));
+  };
+  // the int4 conversion constants live in VGPRs: v_and_or_b32 (VOP3) takes no literal
+  // operands on this architecture and at most one scalar one, so with literals the
+  // conversion would cost two instructions per dword instead of one
+  uint32_t q_mask = 0x000f000fu, q_bias = 0x43004300u;
+  asm volatile("" : "+v"(q_mask), "+v"(q_bias));
+
+  f32x4 acc[RT][PASS / 16];
+  // one step of TT token tiles
+  auto compute = [&](auto tt_c, const Weights& w, int buf) PF_INL {
+    constexpr int TT = decltype(tt_c)::value;
+    // distinct per TT, here and at the end: the variants' common heads and tails must not be merged (merged
+    // heads keep every fragment live at once, merged tails address the sums by a variable index)
+    asm volatile("; %0 token tiles" ::"n"(TT));
+    if constexpr (F::paired) {
+      // min term of the step's four groups as one fp32 MFMA: A = group sums X[token c16][g],
+      // B = (m - 128 s)[row c16][g] (this lane's scale word g); accumulated straight into the sums,
+      // step by step: the min terms cancel most of the 128 q offset of the products, and
+      // summing them apart would lose that cancellation's bits
+      float cg[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const uint32_t lo = pick((g & 1) != 0, w.t[r].sc.y, w.t[r].sc.x), hi = pick((g & 1) != 0, w.t[r].sc.w, w.t[r].sc.z);
+        const float2 sm = F::scale_val(pick(g >= 2, hi, lo));
+        cg[r] = sm.y - 128.f * sm.x;
+      }
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const float xg = *reinterpret_cast<const float*>(lds(ld_s + buf * SLICE * 16 + t * 64));
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xg, cg[r], acc[r][t], 0, 0, 0);
+      }
+      // Lane (c16, g) holds nibbles [32 g, 32 g + 32) of a pair's 128 (g < 2: group A, g >= 2: group
+      // B), word j its inputs + 8 j.  Swapping words 2, 3 of lanes 0..31 with words 0, 1 of lanes
+      // 32..63 (same weight row c16) leaves every lane with two words of each group: A inputs
+      // 8 tb .. 8 tb + 15 and the same of B (tb = 4 (g & 1) + 2 (g >> 1), in 8-input blocks), so
+      // each group takes two full MFMAs against token blocks tb, tb + 1 (A) and tb + 8, tb + 9 (B)
+      // four phases (64-input groups), software pipelined: phase k's MFMAs are followed by the token
+      // reads and the dequantisation of phase k + 1, which run while the matrix unit works
+      struct Frags {
+        uint4 f0[RT], f1[RT], a0[TT], a1[TT];
+        float sc[RT];
+      } fr[2];
+      uint32_t sw[RT][4];  // per tile: words of group A, then of group B
+      auto reads = [&](int k, Frags& f) PF_INL {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          f.a0[t] = tok_frag(buf, t, k >> 1, 2 * (k & 1));
+          f.a1[t] = tok_frag(buf, t, k >> 1, 2 * (k & 1) + 1);
+        }
+      };
+      auto dequant = [&](int k, Frags& f) PF_INL {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          if ((k & 1) == 0) {
+            const uint4 v = w.t[r].raw[k >> 1];
+            const auto s02 = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+            const auto s13 = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+            sw[r][0] = s02[0], sw[r][1] = s13[0], sw[r][2] = s02[1], sw[r][3] = s13[1];
+          }
+          f.f0[r] = q4_frag(sw[r][2 * (k & 1)], q_mask, q_bias);
+          f.f1[r] = q4_frag(sw[r][2 * (k & 1) + 1], q_mask, q_bias);
+          const uint4 s4 = w.t[r].sc;
+          f.sc[r] = F::scale_val(k == 0 ? s4.x : k == 1 ? s4.y : k == 2 ? s4.z : s4.w).x;
+        }
+      };
+      reads(0, fr[0]);
+      dequant(0, fr[0]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        Frags& f = fr[k & 1];
+        const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+        f32x4 u[RT][TT];
+        if (k < 3) reads(k + 1, fr[(k + 1) & 1]);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int r = 0; r < RT; ++r) u[r][t] = mfma(f.a0[t], f.f0[r], z4);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int r = 0; r < RT; ++r) u[r][t] = mfma(f.a1[t], f.f1[r], u[r][t]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (k < 3) dequant(k + 1, fr[(k + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[r][t][i] = __builtin_fmaf(f.sc[r], u[r][t][i], acc[r][t][i]);
+      }
+    } else {
+      // both groups of the step share one scale (applied per group, as in k_grouped); lane (c16, g) holds inputs 16 g .. 16 g + 15
+      uint4 f[RT][4];
+      float sc[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        F::frags(w.t[r].raw[0], f[r][0], f[r][1]);
+        F::frags(w.t[r].raw[1], f[r][2], f[r][3]);
+        sc[r] = F::scale_val(w.t[r].sc).x;
+      }
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const uint4 a0 = tok_frag(buf, t, 0, 0), a1 = tok_frag(buf, t, 0, 1), a2 = tok_frag(buf, t, 0, 2), a3 = tok_frag(buf, t, 0, 3);
+        const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const f32x4 u = mfma(a1, f[r][1], mfma(a0, f[r][0], z4)), v = mfma(a3, f[r][3], mfma(a2, f[r][2], z4));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            acc[r][t][i] = __builtin_fmaf(sc[r], u[i], acc[r][t][i]);
+            acc[r][t][i] = __builtin_fmaf(sc[r], v[i], acc[r][t][i]);
+          }
+        }
+      }
+    }
+    asm volatile("; end of %0 token tiles" ::"n"(TT));
+  };
+  // the item's outputs, through a buffer resource bounded at the pass's last token (stores past it
+  // are dropped)
+  auto finish = [&](const Item& it) PF_INL {
+    if (wave >= AW) return;
+    constexpr int OB = MODE == 0 ? 2 : 4;  // bytes per output
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<char*>(out) + (size_t)it.row0 * NO * OB, 0, it.ntok * NO * OB, 0x00020000);
+#pragma unroll
+    for (int t = 0; t < PASS / 16; ++t) {
+      if (16 * t >= it.ntok) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = (16 * t + 4 * g + i) * NO + it.n0;
+        if constexpr (MODE == 0) {
+          __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(silu(acc[0][t][i]) * acc[1][t][i]), rs, (row + c16) * OB, 0, 0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[r][t][i]), rs, (row + c16) * OB, 64 * r, 0);
+        }
+      }
+    }
+  };
+
+  // items it[0] (computed), it[1], it[2] (requested ahead: DEPTH steps reach SPT >= 4 one, SPT = 2 two items)
+  constexpr int LA = SPT >= DEPTH ? 1 : 2;
+  Item it[LA + 1];
+  int next = LA + 1;
+  items_from(0);
+#pragma unroll
+  for (int k = 0; k <= LA; ++k) it[k] = item_at(k);
+  if (!it[0].valid) return;
+  static_assert(!GATHER || LA == 1, "the row map is read one item ahead");
+  Weights ring[DEPTH];
+  Tok tok[2];  // slices of even / odd parity
+  const int rows0 = rows_of(it[0]);
+  int rows = rows_of(it[LA]);
+  fetch(it[0], 0, ring[0]);
+  offsets_of(it[0], rows0);
+  load_tok(it[0], 0, tok[0]);
+  load_tok(it[0], 1, tok[1]);
+  fetch(it[0], 1, ring[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  store_tok(tok[0], 0, it[0].ntok);
+  load_tok(it[2 / SPT], 2 % SPT, tok[0]);
+  fetch(it[2 / SPT], 2 % SPT, ring[2]);
+  fetch(it[3 / SPT], 3 % SPT, ring[3]);
+  __builtin_amdgcn_sched_barrier(0);
+  lds_barrier();
+  // one item whose first step uses ring slot S0; false after the block's last item
+  auto run_item = [&](auto s0_c) PF_INL {
+    constexpr int S0 = decltype(s0_c)::value;
+    const int tiles = (it[0].ntok + 15) >> 4;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int t = 0; t < PASS / 16; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int RND = SPT < DEPTH ? SPT : DEPTH;  // steps per round
+#pragma unroll 1
+    for (int i0 = 0; i0 < SPT; i0 += RND) {
+      // the item and step that lie DEPTH steps ahead of this round's first step
+      const bool same = i0 + DEPTH < SPT;
+      const int f0 = same ? i0 + DEPTH : 0;
+      Item fi;
+      fi.wq = pick(same, it[0].wq, it[LA].wq), fi.ws = pick(same, it[0].ws, it[LA].ws);
+      fi.row0 = pick(same, it[0].row0, it[LA].row0), fi.ntok = pick(same, it[0].ntok, it[LA].ntok);
+      fi.n0 = pick(same, it[0].n0, it[LA].n0), fi.valid = true;
+#pragma unroll
+      for (int d = 0; d < RND; ++d) {
+        Weights& w = ring[(S0 + d) % DEPTH];
+        switch (tiles) {
+          case 1: compute(std::integral_constant<int, 1>{}, w, d & 1); break;
+          case 2: compute(std::integral_constant<int, 2>{}, w, d & 1); break;
+          case 3:
+            if constexpr (PASS > 32) compute(std::integral_constant<int, 3>{}, w, d & 1);
+            break;
+          default:
+            if constexpr (PASS > 48) compute(std::integral_constant<int, 4>{}, w, d & 1);
+            break;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        store_tok(tok[(d + 1) & 1], (d + 1) & 1, pick(d + 1 < RND || i0 + RND < SPT, it[0].ntok, it[1].ntok));
+        __builtin_amdgcn_sched_barrier(0);
+        if (d == 0) {  // slice DEPTH - 1 counted from this round's first, then those of fi
+          if constexpr (SPT < DEPTH) load_tok(it[1], DEPTH - 1 - SPT, tok[1]);
+          else load_tok(it[0], i0 + DEPTH - 1, tok[1]);
+          if (!same) offsets_of(it[LA], rows);
+        } else {
+          load_tok(fi, f0 + d - 1, tok[(d + 1) & 1]);
+        }
+        fetch(fi, f0 + d, w);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();
+      }
+    }
+    finish(it[0]);
+    if (!it[1].valid) return false;
+#pragma unroll
+    for (int k = 0; k < LA; ++k) it[k] = it[k + 1];
+    it[LA] = item_at(next++), rows = rows_of(it[LA]);
+    return true;
+  };
+  for (;;) {
+    if (!run_item(std::integral_constant<int, 0>{})) break;
+    if constexpr (NI == 2) {
+      if (!run_item(std::integral_constant<int, SPT % DEPTH>{})) break;
+    }
+  }
 }
 
 
@@ -914,40 +1371,54 @@ inline int resident_blocks(const void* kern, int threads, size_t lds) {
   return v;
 }
 
+// k_grouped_pass from 14 top-8 picks per expert on (448 token rows at 256 experts), where experts with a
+// second 16-token pass become common.  Whole prefill layers at 256 experts, k_grouped ->
+// k_grouped_pass: int4 300 rows 147 -> 150 us, 449 rows 173 -> 174, 512 (reference layout) 201 -> 194, 1024
+// 303 -> 264, hot experts 460 / 900 rows 170 / 249 -> 160 / 223; fp8 12 rows 94 -> 104, 300 rows 203 -> 207,
+// 460 rows 226 -> 227, 600 rows 258 -> 243.  The number of rows is only known where they come through
+// a row map; elsewhere (x_rows 0) k_grouped stays.
+inline bool use_passes(int x_rows, int E) { return (long long)x_rows * 8 >= 14ll * E; }
+
 template <class F>
 void launch_grouped(const uint8_t* wq, const void* ws, const uint16_t* X, const int* offsets, const int* counts,
                     void* out, int E, int N, int K, int mode, size_t eq, size_t es, int sb, int fixed_rows,
                     hipStream_t st, const int* rmap = nullptr, int x_rows = 0, bool packed = false) {
-  const int rows_out = mode == 0 ? N / 2 : N;
-  if (fixed_rows >= 0) {
+  if constexpr (F::q8) {
     // one weight set over all rows (the shared expert).  gate_up: the K-split kernel, one
     // 16-row tile per block, token tiles over grid z (z = 4, 16, 32 and the dense kernel measured
     // slower); down: the dense weight-stationary kernel (6.6 against 10.2 us at 300 rows)
     if (mode == 0) {
       const int tiles = (fixed_rows + PF_TOK - 1) / PF_TOK;
-      const dim3 grid(1, rows_out / 16, tiles < 8 ? tiles : 8);
+      const dim3 grid(1, N / 2 / 16, tiles < 8 ? tiles : 8);
       hipLaunchKernelGGL((k_grouped_ks<F, 0, 2048>), grid, dim3(PF_WPB * 64), 0, st, wq, ws, X, offsets, counts, out,
                          N, eq, es, sb, fixed_rows);
-    } else if constexpr (F::q8) {  // fixed_rows is the int8 shared expert's mode only
+    } else {
       const dim3 grid((fixed_rows + DQ_TM - 1) / DQ_TM, N / 32);
       hipLaunchKernelGGL((k_dense_q8<typename F::Scale, 512>), grid, dim3(256), 32 * (512 + 16) + 4096, st, wq,
                          reinterpret_cast<const uint16_t*>(ws), X, reinterpret_cast<float*>(out), fixed_rows, N);
     }
-    return;
+  } else {
+    // grouped experts: a persistent grid of as many blocks as are resident at once, walking the
+    // work items (expert, token pass, row block) the kernel derives from counts
+    const dim3 block(PF_GWPB * 64);
+    if (use_passes(x_rows, E)) {
+      auto kern = packed ? (mode == 1 ? k_grouped_pass<F, 1, 512, false, true>
+                                      : rmap ? k_grouped_pass<F, 0, 2048, true, true> : k_grouped_pass<F, 0, 2048, false, true>)
+                         : (mode == 1 ? k_grouped_pass<F, 1, 512, false, false>
+                                      : rmap ? k_grouped_pass<F, 0, 2048, true, false> : k_grouped_pass<F, 0, 2048, false, false>);
+      hipLaunchKernelGGL(kern, dim3(resident_blocks((const void*)kern, PF_GWPB * 64, 0)), block, 0, st, wq, ws, X,
+                         offsets, counts, out, N, eq, es, sb, E, rmap, x_rows);
+      return;
+    }
+    const size_t lds = 2 * ((size_t)PF_TOK * K * 2 + (F::paired ? (size_t)(K / 64) * PF_TOK * 4 : 0)) + 192 * 16 +
+                       (mode == 0 ? 2 * PF_GRPW * (PF_GWPB / 2) * 64 * 16 : 0);
+    auto kern = packed ? (mode == 1 ? k_grouped<F, 1, 512, false, true>
+                                    : rmap ? k_grouped<F, 0, 2048, true, true> : k_grouped<F, 0, 2048, false, true>)
+                       : (mode == 1 ? k_grouped<F, 1, 512, false, false>
+                                    : rmap ? k_grouped<F, 0, 2048, true, false> : k_grouped<F, 0, 2048, false, false>);
+    hipLaunchKernelGGL(kern, dim3(resident_blocks((const void*)kern, PF_GWPB * 64, lds)), block, lds, st, wq, ws, X,
+                       offsets, counts, out, N, eq, es, sb, E, err_word(), rmap, x_rows);
   }
-  // grouped experts: a persistent grid of as many blocks as are resident at once, walking the
-  // work items (expert, token pass, row block) the kernel derives from counts
-  const size_t lds = 2 * ((size_t)PF_TOK * K * 2 + (F::paired ? (size_t)(K / 64) * PF_TOK * 4 : 0)) + 192 * 16 +
-                     (mode == 0 ? 2 * PF_GRPW * (PF_GWPB / 2) * 64 * 16 : 0);
-  auto kern = mode == 1 ? k_grouped<F, 1, 512, false> : rmap ? k_grouped<F, 0, 2048, true> : k_grouped<F, 0, 2048, false>;
-  if constexpr (F::packable) {
-    if (packed)
-      kern = mode == 1 ? k_grouped<F, 1, 512, false, true>
-                       : rmap ? k_grouped<F, 0, 2048, true, true> : k_grouped<F, 0, 2048, false, true>;
-  }
-  int grid = resident_blocks((const void*)kern, PF_GWPB * 64, lds);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(PF_GWPB * 64), lds, st, wq, ws, X, offsets, counts, out, N, eq, es, sb, E,
-                     err_word(), rmap, x_rows);
 }
 
 // gate_up then down for all experts of a grouped batch; with rmap, the gate_up token rows are
@@ -961,7 +1432,7 @@ int moe_prefill(const uint8_t* gu_q, const void* gu_s, const uint8_t* d_q, const
   if (rmap && (x_rows < 1 || (long long)x_rows * H * 2 > 0x7fffffffll)) return -1;
   launch_grouped<F>(gu_q, gu_s, xp, offsets, counts, act, E, 2 * I, H, 0, gu_q_b, gu_s_e, sb, -1, st, rmap, x_rows,
                     packed);
-  launch_grouped<F>(d_q, d_s, act, offsets, counts, y, E, H, I, 1, d_q_b, d_s_e, sb, -1, st, nullptr, 0, packed);
+  launch_grouped<F>(d_q, d_s, act, offsets, counts, y, E, H, I, 1, d_q_b, d_s_e, sb, -1, st, nullptr, x_rows, packed);
   return 0;
 }
 

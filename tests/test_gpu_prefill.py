@@ -613,3 +613,54 @@ def test_prefill_rows_packed_fp8_matches(fmt, skew, E, rows):
         outs.append((host(act), host(yp)))
     np.testing.assert_array_equal(outs[1][0], outs[0][0])
     np.testing.assert_array_equal(outs[1][1].view(np.uint32), outs[0][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,fmt,packed", [("q4", "ref", False), ("q4", "cfg", True), ("fp8", "ref", True),
+                                             ("fp8", "cfg", False)])
+@pytest.mark.parametrize("counts", [
+    [1, 0, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 96, 129],  # edges of token tiles and of passes
+    [14, 0, 0, 0, 0, 0, 0, 0],                                        # fewer items than blocks
+    [17000] * 8,                                                      # more than 64 items per block
+])
+def test_prefill_passes_match_tiles(kind, fmt, packed, counts):
+    """The kernel of the larger token counts (dr_moe_prefill_rows* from 14 top-8 picks per expert on) gives
+    the act and y bits of the kernel of the smaller ones (dr_moe_prefill*, whose rows are gathered, at
+    every count), with token rows in any order."""
+    import torch
+
+    E, n = len(counts), sum(counts)
+    lib, P, st = D.lib(), D.ptr, D.stream_ptr()
+    g = torch.Generator(device="cuda").manual_seed(n + E)
+    L = {k: dev(v) for k, v in synth.make_layer(43, E=E, fmt=fmt, kind=kind, quick=True).items()
+         if k in ("gu_q", "gu_s", "d_q", "d_s")}
+    W = dict(L)
+    if packed:
+        for q, s, nn, kk in (("gu_q", "gu_s", 2 * I, H), ("d_q", "d_s", H, I)):
+            W[q] = torch.zeros_like(L[q])
+            if kind == "q4":
+                W[s] = torch.zeros_like(L[s])
+                lib.dr_moe_pack_q4(P(L[q]), P(L[s]), E, nn, kk, P(W[q]), P(W[s]), st)
+            else:
+                lib.dr_moe_pack_fp8(P(L[q]), E, nn, kk, P(W[q]), st)
+    x = torch.randn(n, H, generator=g, device="cuda").to(torch.bfloat16)
+    ros = torch.randint(0, n, (n + 16,), generator=g, device="cuda", dtype=torch.int32)
+    cnt = torch.tensor(counts, dtype=torch.int32, device="cuda")
+    off = (torch.cumsum(cnt, 0) - cnt).to(torch.int32)
+    sfx = ("_fp8" if kind == "fp8" else "") + ("_bf16s" if fmt == "cfg" else "")
+    outs = []
+    for rows in (True, False):
+        act = torch.zeros(n, I, dtype=torch.int16, device="cuda")
+        y = torch.zeros(n, H, device="cuda")
+        if rows:
+            getattr(lib, "dr_moe_prefill_rows" + ("_packed" if packed else "") + sfx)(
+                P(W["gu_q"]), P(W["gu_s"]), P(W["d_q"]), P(W["d_s"]), P(x), n, P(ros), P(off), P(cnt), P(act), P(y), E,
+                H, I, st)
+        else:
+            xp = x[ros[:n].long()].contiguous()
+            getattr(lib, "dr_moe_prefill" + sfx)(P(L["gu_q"]), P(L["gu_s"]), P(L["d_q"]), P(L["d_s"]), P(xp), P(off),
+                                                 P(cnt), P(act), P(y), E, H, I, st)
+        torch.cuda.synchronize()
+        outs.append((act, y.view(torch.int32)))
+    assert lib.dr_last_error() == 0
+    assert outs[0][1].any()
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
