@@ -62,10 +62,10 @@ __global__ void __launch_bounds__(320)
   }
 }
 
-// The same canonical GEMM for few rows of A (M <= GR_MAXM, decode batches): one wave per W
-// row, which it loads once and dots with every A row (4 at a time, all loads issued first);
-// 8 waves per block.  Every dot has the canonical order, so C equals k_gemm_tile's bits.
-constexpr int GR_MAXM = 16;
+// The canonical GEMM for up to 4 rows of A (decode batches): one wave per W row, which it loads once and
+// dots with every A row (all loads issued first); 8 waves per block.  3.8 us at 4 x 257 x 2048 against
+// 5.1 for k_gemm_mfma, whose 16-row tiles would be mostly empty (5 rows: 5.3 against 4.9).
+constexpr int GR_MAXM = 4;
 template <int NCH>
 __global__ void __launch_bounds__(512)
     k_gemm_rows(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, float* __restrict__ C, int M,
@@ -118,124 +118,154 @@ __global__ void __launch_bounds__(512)
   }
 }
 
-// The same canonical GEMM, one wave per 8 x 8 tile of C (4 tiles per block, no LDS): lane l
-// accumulates all 64 dots over its chunks l + 64 j in element order (the canonical lane sums),
-// then one reduce-scatter over the ascending xor tree finishes them together.  Step o pairs
-// lane l with l ^ o exactly as the canonical butterfly does, and each pair of lanes splits its
-// list of partial sums: the lane with bit o clear keeps the first half (adding its partner's
-// copy of it), the other the second half, so after the six steps lane l holds output
-// bitrev6(l) with the canonical tree's bits (a + b = b + a).  Exchanges: DPP quad_perm (o = 1,
-// 2) and row_ror (o = 4: by 12 for the lanes whose partner is l + 4, by 4 for l - 4; o = 8: by
-// 8), v_permlane16_swap / v_permlane32_swap (o = 16, 32; the swap itself hands each lane the
-// half it keeps).  A and W chunks of the next j are requested before the current j's FMAs.
-// Measured at 300 x 257 x 2048 with 8 x 8 tiles: 12.0 us (a 2 x 8 per-wave kernel with one butterfly
-// per dot: 16.8 us); 4 x 8 tiles (twice the waves, more conversions per FMA) 13.9 us.
-template <int O, int V>
-DEV void rs_step(float (&v)[64]) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int k = 0; k < V / 2; ++k) {
-    const float x = v[k], y = v[k + V / 2];
-    if constexpr (O >= 16) {
-      const auto r = O == 16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false)
-                             : __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-      v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    } else {
-      constexpr int cx = O == 1 ? 0xB1 : O == 2 ? 0x4E : O == 4 ? 0x12C : 0x128;
-      constexpr int cy = O == 1 ? 0xB1 : O == 2 ? 0x4E : O == 4 ? 0x124 : 0x128;
-      const float px = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), cx, 0xF, 0xF, true));
-      const float py = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y), cy, 0xF, 0xF, true));
-      v[k] = (lane & O) ? y + py : x + px;
-    }
-  }
-}
-
-// Tiles of TM x TN outputs (at most 8 x 8: the 64 reduce-scatter slots; the unused slots stay
-// zero and are never stored).  8 x 5 balances 300 x 257 best over the 1024 SIMDs: measured 9.5-9.8
-// us against 10.7-11.2 for 8 x 8 (1254 tiles, a fifth of the SIMDs running two), 9.8 for 8 x 6,
-// 10.1-10.3 for 8 x 7 and 12.1 for 8 x 4 (more A loads per FMA), with identical bits.
-constexpr int GT_TM = 8, GT_TN = 5;
-template <int NCH, int TM = GT_TM, int TN = GT_TN>
-__global__ void __launch_bounds__(256)
-    k_gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, float* __restrict__ C, int M, int N,
+// The same canonical GEMM on the fp32 matrix unit.  v_mfma_f32_16x16x1_4b_f32 is four independent 16 x 16
+// rank-1 updates whose every element is one fp32 fma (rounded to nearest even, subnormals kept, checked
+// against fmaf), so block b of an instruction can carry the running sum of one canonical lane: set s
+// of a wave holds lanes 4 s .. 4 s + 3 of the 64 as the four blocks, and inputs enter in the canonical
+// order (chunk lane + 64 j, then element).  An MFMA lane (b, i) reads whole 16-byte chunks of row i, 8
+// MFMAs per chunk pair, straight from global memory.  The four blocks of an output lie in one
+// lane's registers, so the canonical xor tree is (b0 + b1) + (b2 + b3) there, then over the wave's
+// sets, then over the NW waves through LDS (a + b = b + a, so the same bits as the butterfly).
+// The matrix unit does 32 of these fmas per clock and SIMD where the vector unit does 16, and
+// the bf16 -> fp32 conversions fall from one per 8 / 5 fmas to one per 16 and matrix row.
+// Block: 16 BM x 16 BN outputs, NW waves of 64 / NW canonical lanes each.  Consecutive tiles of
+// one XCD share their W rows.
+// What bounds it: large shapes the loads (16 rows x 64 bytes per instruction, ~8 TB/s of L2 reads; 32 x 32
+// tiles run at 65% of the fp32 matrix rate), small ones the 2048-long chains of one tile (7 us per 32 x 32).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <int NCH, int BM, int BN, int NW, bool FULL>
+__global__ void __launch_bounds__(NW * 64)
+    k_gemm_mfma(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, float* __restrict__ C, int M, int N,
                 int K, float beta) {
-#pragma clang fp contract(off)
-  static_assert(TM >= 1 && TM <= 8 && TN >= 1 && TN <= 8, "tile of at most 8 x 8 (64 reduce-scatter slots)");
-  const int lane = lane_id();
-  const int tn = (N + TN - 1) / TN;
-  const int tile = blockIdx.x * 4 + wave_id();
-  const int m0 = (tile / tn) * TM, n0 = (tile % tn) * TN;
-  if (m0 >= M) return;
-  const int KC = K / 8;
-  const uint16_t* ap[8];
-  const uint16_t* wp[8];
+  constexpr int S = 16 / NW;               // sets of four canonical lanes per wave
+  constexpr int D = NCH < 2 ? NCH : 2;     // chunk rounds in flight
+  __shared__ float red[NW][BM * BN * 4][64];
+  const int lane = lane_id(), wave = wave_id(), i16 = lane & 15;
+  const int tm = (M + 16 * BM - 1) / (16 * BM), tiles = tm * ((N + 16 * BN - 1) / (16 * BN));
+  const int per = (tiles + 7) / 8, tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (tile >= tiles) return;
+  const int m0 = tile % tm * 16 * BM, n0 = tile / tm * 16 * BN;
+  const int KC = K / 8, c0 = 64 / NW * wave + (lane >> 4);  // this lane's first chunk
+  const uint16_t *ap[BM], *wp[BN];  // rows past the end repeat the last one; their outputs are not stored
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    ap[r] = A + (size_t)(m0 + r < M ? m0 + r : M - 1) * K + (size_t)lane * 8;
-    wp[r] = W + (size_t)(n0 + r < N ? n0 + r : N - 1) * K + (size_t)lane * 8;
-  }
-  (void)ap, (void)wp;
-  float acc[64];
+  for (int x = 0; x < BM; ++x) ap[x] = A + (size_t)min(m0 + 16 * x + i16, M - 1) * K;
 #pragma unroll
-  for (int i = 0; i < 64; ++i) acc[i] = 0.f;
-  uint4 ac[2][8], wc[2][8];
-  auto load = [&](int j, int b) {
-    const bool in = lane + WAVE * j < KC;
+  for (int y = 0; y < BN; ++y) wp[y] = W + (size_t)min(n0 + 16 * y + i16, N - 1) * K;
+  f32x16 acc[S][BM][BN];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      if (r < TM) ac[b][r] = in ? ld16(ap[r] + (size_t)j * WAVE * 8) : make_uint4(0, 0, 0, 0);
-      if (r < TN) wc[b][r] = in ? ld16(wp[r] + (size_t)j * WAVE * 8) : make_uint4(0, 0, 0, 0);
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int x = 0; x < BM; ++x)
+#pragma unroll
+      for (int y = 0; y < BN; ++y) acc[s][x][y] = (f32x16)(0.f);
+  uint4 av[D][S][BM], wv[D][S][BN];
+  // FULL: every chunk exists (K = 512 NCH); otherwise chunks past K / 8 are zero (fma(0, 0, sum) = sum)
+  auto chunk = [&](const uint16_t* row, int c) {
+    const uint4 v = ld16(row + (size_t)(FULL ? c : min(c, KC - 1)) * 8);
+    return FULL || c < KC ? v : make_uint4(0, 0, 0, 0);
+  };
+  auto load = [&](int j) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+      for (int x = 0; x < BM; ++x) av[j % D][s][x] = chunk(ap[x], c0 + 4 * s + 64 * j);
+#pragma unroll
+      for (int y = 0; y < BN; ++y) wv[j % D][s][y] = chunk(wp[y], c0 + 4 * s + 64 * j);
     }
   };
-  load(0, 0);
+#pragma unroll
+  for (int j = 0; j < D; ++j) load(j);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    const int b = j & 1;
-    if (j + 1 < NCH) load(j + 1, b ^ 1);
-    if (lane + WAVE * j < KC) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float a[8], w[8];
+        auto element = [&](const uint4& v) {
+          const uint32_t q = e < 2 ? v.x : e < 4 ? v.y : e < 6 ? v.z : v.w;
+          return (e & 1) ? bf16_hi(q) : bf16_lo(q);
+        };
+        float a[BM], w[BN];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          if (r < TM) {
-            const uint32_t aw = e < 2 ? ac[b][r].x : e < 4 ? ac[b][r].y : e < 6 ? ac[b][r].z : ac[b][r].w;
-            a[r] = (e & 1) ? bf16_hi(aw) : bf16_lo(aw);
-          }
-          if (r < TN) {
-            const uint32_t ww = e < 2 ? wc[b][r].x : e < 4 ? wc[b][r].y : e < 6 ? wc[b][r].z : wc[b][r].w;
-            w[r] = (e & 1) ? bf16_hi(ww) : bf16_lo(ww);
-          }
+        for (int x = 0; x < BM; ++x) a[x] = element(av[j % D][s][x]);
+#pragma unroll
+        for (int y = 0; y < BN; ++y) w[y] = element(wv[j % D][s][y]);
+#pragma unroll
+        for (int x = 0; x < BM; ++x)
+#pragma unroll
+          for (int y = 0; y < BN; ++y)
+            acc[s][x][y] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[x], w[y], acc[s][x][y], 0, 0, 0);
+      }
+    if (j + D < NCH) load(j + D);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // D layout: register 4 b + r of lane l is row 4 (l / 16) + r, column l % 16 of block b
+#pragma unroll
+  for (int x = 0; x < BM; ++x)
+#pragma unroll
+    for (int y = 0; y < BN; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float p[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const f32x16& v = acc[s][x][y];
+          p[s] = (v[r] + v[4 + r]) + (v[8 + r] + v[12 + r]);
         }
 #pragma unroll
-        for (int m = 0; m < TM; ++m)
+        for (int d = 1; d < S; d *= 2)
 #pragma unroll
-          for (int n = 0; n < TN; ++n) acc[8 * m + n] = __builtin_fmaf(w[n], a[m], acc[8 * m + n]);
+          for (int s = 0; s + d < S; s += 2 * d) p[s] = p[s] + p[s + d];
+        red[wave][(x * BN + y) * 4 + r][lane] = p[0];
       }
+  __syncthreads();
+  for (int o = wave; o < BM * BN * 4; o += NW) {
+    float p[NW];
+#pragma unroll
+    for (int q = 0; q < NW; ++q) p[q] = red[q][o][lane];
+#pragma unroll
+    for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+      for (int q = 0; q + d < NW; q += 2 * d) p[q] = p[q] + p[q + d];
+    const int m = m0 + 16 * (o / (4 * BN)) + 4 * (lane >> 4) + (o & 3), n = n0 + 16 * (o / 4 % BN) + i16;
+    if (m < M && n < N) {
+      float* c = C + (size_t)m * N + n;
+      *c = beta == 0.f ? p[0] : p[0] + beta * *c;
     }
-  }
-  rs_step<1, 64>(acc);
-  rs_step<2, 32>(acc);
-  rs_step<4, 16>(acc);
-  rs_step<8, 8>(acc);
-  rs_step<16, 4>(acc);
-  rs_step<32, 2>(acc);
-  const int i = (int)(__builtin_bitreverse32((uint32_t)lane) >> 26);
-  const int m = m0 + (i >> 3), n = n0 + (i & 7);
-  if ((i >> 3) < TM && (i & 7) < TN && m < M && n < N) {
-    float* c = C + (size_t)m * N + n;
-    *c = beta == 0.f ? acc[0] : acc[0] + beta * *c;
   }
 }
 
+template <int NCH, int BM, int BN, int NW>
+void launch_gemm_mfma(const uint16_t* A, const uint16_t* W, float* C, int M, int N, int K, float beta, hipStream_t st) {
+  const int tiles = ((M + 16 * BM - 1) / (16 * BM)) * ((N + 16 * BN - 1) / (16 * BN));
+  const dim3 grid((tiles + 7) / 8 * 8), block(NW * 64);
+  if (K == NCH * 512)
+    hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, true>), grid, block, 0, st, A, W, C, M, N, K, beta);
+  else
+    hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, false>), grid, block, 0, st, A, W, C, M, N, K, beta);
+}
+
+// The largest tile whose blocks still fit the 256 CUs at once (a block's time is its tile's), us at K = 2048
+// for 16 x 16, 32 x 16 (16 waves), 32 x 32 tiles: 100 x 257 5.8 / 8.1 / 12.0, 300 x 257 9.6 / 8.6 / 12.3,
+// 512 x 257 13.6 / 15.3 / 12.6.  Past one round of 32 x 32 tiles, two 8-wave blocks of 32 x 16 per CU
+// (1024 x 257 24.4 -> 21.2, 300 x 1024 24.1 -> 21.3; K = 512: 300 x 2048 13.2 -> 11.7) until a second round of 32 x 32
+// tiles is well filled (512 x 1024 28.0 -> 25.1).  The vector kernel this replaces (8 x 5 outputs per wave):
+// 6.9 us at 100 x 257, 8.5 at 300, 15.3 at 512, 28.0 at 1024, 49.7 at 512 x 1024, 26.4 at 512 x 2048 x 512.
 template <int NCH>
 void launch_gemm(const uint16_t* A, const uint16_t* W, float* C, int M, int N, int K, float beta, hipStream_t st) {
-  if (M <= GR_MAXM) {
+  constexpr long long CUS = 256;
+  const long long m16 = (M + 15ll) / 16, m32 = (M + 31ll) / 32, n16 = (N + 15ll) / 16, n32 = (N + 31ll) / 32;
+  if (M <= GR_MAXM)
     hipLaunchKernelGGL(k_gemm_rows<NCH>, dim3((N + 7) / 8), dim3(512), 0, st, A, W, C, M, N, K, beta);
-    return;
-  }
-  const int tiles = ((M + GT_TM - 1) / GT_TM) * ((N + GT_TN - 1) / GT_TN);
-  hipLaunchKernelGGL(k_gemm_tile<NCH>, dim3((tiles + 3) / 4), dim3(256), 0, st, A, W, C, M, N, K, beta);
+  else if (m16 * n16 <= CUS)
+    launch_gemm_mfma<NCH, 1, 1, 16>(A, W, C, M, N, K, beta, st);
+  else if (m32 * n16 <= CUS)
+    launch_gemm_mfma<NCH, 2, 1, 16>(A, W, C, M, N, K, beta, st);
+  else if (m32 * n32 <= CUS || (K > 512 && 2 * m32 * n32 > 3 * CUS))
+    launch_gemm_mfma<NCH, 2, 2, 16>(A, W, C, M, N, K, beta, st);
+  else
+    launch_gemm_mfma<NCH, 2, 1, 8>(A, W, C, M, N, K, beta, st);
 }
 
 }  // namespace

@@ -177,3 +177,45 @@ def test_router_nan_input_selects_valid_experts():
     gi = host(idx)
     assert len(set(gi.tolist())) == 8 and gi.min() >= 0 and gi.max() < E
     np.testing.assert_array_equal(gi, ri)
+
+
+@pytest.mark.parametrize("M,N,K,beta", [
+    (4, 33, 2048, 0.0), (5, 17, 2048, 1.0),          # the vector kernel's last size, 16 x 16 tiles with ragged edges
+    (250, 257, 8, 0.0), (260, 257, 2048, 0.5),       # one chunk; 32 x 16 tiles, 16 waves
+    (500, 261, 520, 0.0), (290, 1000, 2048, 0.0),    # 32 x 32 tiles, chunks past K; 32 x 16 tiles, 8 waves
+    (330, 1200, 1000, 1.0), (530, 700, 512, 0.0),    # a second round of 32 x 32 tiles; K = 512
+    (40, 70, 4096, 0.0),
+])
+def test_gemm_matrix_unit_bit_exact(M, N, K, beta):
+    """dr_gemm's fp32 matrix-unit tiles against the canonical order at every tile shape, with subnormal
+    products, signed zeros and infinities among the inputs, and C read through beta."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    a = rng.normal(0, 1, (M, K)).astype(np.float32)
+    w = rng.normal(0, 0.02, (N, K)).astype(np.float32)
+    a[0] *= 1e-25
+    w[0] *= 1e-15  # subnormal products in C[0, 0]
+    a[1, : K // 2] = -0.0
+    if M > 4:
+        a[3, 0] = np.inf
+    A, Wt = synth.f32_to_bf16(a), synth.f32_to_bf16(w)
+    with np.errstate(invalid="ignore"):
+        ref = O.router_logits_rows(A, Wt, M, N, K)
+    c0 = rng.normal(0, 1, (M, N)).astype(np.float32)
+    C = dev(c0.copy())
+    h = np.zeros(1, np.uint64)
+    L = D.lib()
+    L.dr_cublas_create(h.ctypes.data, D.stream_ptr())
+    dA, dWt = dev(A), dev(Wt)
+    L.dr_gemm(int(h[0]), D.ptr(dA), D.ptr(dWt), D.ptr(C), M, N, K, beta)
+    torch.cuda.synchronize()
+    L.dr_cublas_destroy(int(h[0]))
+    want = np.asarray(ref, np.float32).reshape(M, N)
+    if beta:
+        with np.errstate(invalid="ignore"):
+            want = want + np.float32(beta) * c0
+    got = host(C).reshape(M, N)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    np.testing.assert_array_equal(bits(got[ok]), bits(want[ok]))
