@@ -231,10 +231,13 @@ __global__ void __launch_bounds__(WPB * 64)
 
 // Launch shapes: batch 1 (the engine's per-layer chain) uses 256-thread blocks, many of them;
 // B > 1 uses 512-thread blocks, two per CU (as the FP8 kernels).
-template <class SC, class SH, int B>
+// GB: routed blocks per group.  Every block first stages its group's rows (norm, digits: ~3 us), so with
+// several groups to fill the chip each takes fewer blocks of more units (launch_decode): 20 rows 115 us at 512,
+// 108 at 256; 64 rows 331 / 306 / 296 at 512 / 256 / 128; a single group needs all 512 (two blocks per CU).
+template <class SC, class SH, int B, int GB = 512>
 void launch_gate_up_b(const uint8_t* gu_q, const void* gu_sm, const int8_t* sgu_q, const uint16_t* sgu_s, const float* x,
                       const int* idx, float* act, const float* nw, float eps, int groups, hipStream_t st) {
-  constexpr int GW = B == 1 ? 4 : 8, GB = 512, GD = 2, GS = B == 1 ? 1 : 2;
+  constexpr int GW = B == 1 ? 4 : 8, GD = 2, GS = B == 1 ? 1 : 2;
   constexpr int NB = GB + DEC_I / (GW * GS);
   hipLaunchKernelGGL((k_moe_gate_up_q4<SC, SH, GW, GB, GD, GS, B>), dim3(NB, groups), dim3(GW * 64), 0, st, gu_q,
                      (const uint32_t*)gu_sm, sgu_q, sgu_s, x, idx, act, nw, eps);
@@ -243,7 +246,7 @@ void launch_gate_up_b(const uint8_t* gu_q, const void* gu_sm, const int8_t* sgu_
 // rows independent decode rows (x, res, y: [rows, H]; idx, wts: [rows, topk]; act: rows x
 // (topk + 1) x I).  gate_up: the groups of 4 rows in one launch, the remaining 1 .. 3 rows in a second one;
 // down: one launch.  A pair of launches per 4 rows leaves the chip half idle at every boundary:
-// 20 rows (router included) 162 us that way, 115 now; 64 rows 504 -> 331.
+// 20 rows (router included) 162 us that way, 108 now; 64 rows 504 -> 296.
 template <class SC, class SH>
 int launch_decode(const uint8_t* gu_q, const void* gu_sm, const uint8_t* d_q, const void* d_sm, const int8_t* sgu_q,
                   const uint16_t* sgu_s, const int8_t* sd_q, const uint16_t* sd_s, const float* x, const int* idx,
@@ -255,7 +258,9 @@ int launch_decode(const uint8_t* gu_q, const void* gu_sm, const uint8_t* d_q, co
   const float* xr = x + (size_t)r0 * H;
   const int* ir = idx + (size_t)r0 * topk;
   float* ar = act + (size_t)r0 * (topk + 1) * I;
-  if (r0) launch_gate_up_b<SC, SH, 4>(gu_q, gu_sm, sgu_q, sgu_s, x, idx, act, nw, eps, r0 / 4, st);
+  if (r0 == 4) launch_gate_up_b<SC, SH, 4>(gu_q, gu_sm, sgu_q, sgu_s, x, idx, act, nw, eps, 1, st);
+  else if (r0 && r0 < 32) launch_gate_up_b<SC, SH, 4, 256>(gu_q, gu_sm, sgu_q, sgu_s, x, idx, act, nw, eps, r0 / 4, st);
+  else if (r0) launch_gate_up_b<SC, SH, 4, 128>(gu_q, gu_sm, sgu_q, sgu_s, x, idx, act, nw, eps, r0 / 4, st);
   if (rem == 1) launch_gate_up_b<SC, SH, 1>(gu_q, gu_sm, sgu_q, sgu_s, xr, ir, ar, nw, eps, 1, st);
   else if (rem == 2) launch_gate_up_b<SC, SH, 2>(gu_q, gu_sm, sgu_q, sgu_s, xr, ir, ar, nw, eps, 1, st);
   else if (rem == 3) launch_gate_up_b<SC, SH, 3>(gu_q, gu_sm, sgu_q, sgu_s, xr, ir, ar, nw, eps, 1, st);

@@ -249,3 +249,31 @@ def test_routed_fp8_rows_equal_three_launch_path(fmt, rows, E):
     del Ld
     torch.cuda.empty_cache()
 
+
+
+@pytest.mark.parametrize("fmt,rows", [("cfg", 7), ("ref", 8), ("cfg", 31), ("ref", 32), ("cfg", 33), ("ref", 64)])
+def test_decode_rows_groups_match_calls_of_four(fmt, rows):
+    """One call over several groups of 4 rows (and a remainder) gives the bits of a call per group,
+    with y written over x."""
+    import torch
+
+    E = 24
+    L = synth.make_layer(250 + rows, E=E, fmt=fmt, quick=True)
+    rng = np.random.default_rng(251 + rows)
+    x = rng.normal(0, 1, (rows, H)).astype(np.float32)
+    idx, wts, sg = _routing(rng, rows, E)
+    t = {k: dev(L[k]) for k in ("gu_q", "gu_s", "d_q", "d_s", "sgu_q", "sgu_s", "sd_q", "sd_s", "nw")}
+    P = D.ptr
+    w8 = [P(t[k]) for k in ("gu_q", "gu_s", "d_q", "d_s", "sgu_q", "sgu_s", "sd_q", "sd_s")]
+    f = getattr(D.lib(), "dr_moe_decode_rows" + ("_bf16s" if fmt == "cfg" else ""))
+    yb = (None,) if fmt == "cfg" else ()
+    act = torch.zeros(rows * (TOPK + 1) * I, device="cuda")
+    out = []
+    for step in (rows, 4):
+        dx, didx, dwts, dsg = dev(x), dev(idx), dev(wts), dev(sg)
+        for r in range(0, rows, step):
+            f(*w8, P(dx[r:]), P(didx[r:]), P(dwts[r:]), P(dsg[r:]), P(dx[r:]), P(act), P(dx[r:]), *yb,
+              min(step, rows - r), H, I, TOPK, P(t["nw"]), 1e-6, D.stream_ptr())
+        torch.cuda.synchronize()
+        out.append(bits(host(dx)))
+    np.testing.assert_array_equal(out[0], out[1])
