@@ -1,4 +1,4 @@
-// Decode router for B rows (B <= 8) as one block's work: shared by dr_router_topk (B = 1),
+// Decode router for B rows (B <= 4) as one block's work: shared by dr_router_topk (B = 1),
 // dr_router_topk_rows (a launch of router blocks only) and the fused small-batch FP8 kernel
 // (router blocks ahead of the gate_up blocks in one launch).  Reference semantics:
 // kernels/drama.cu:317-461 per row.
@@ -10,17 +10,16 @@
 // of canon.hpp, so each row's logits, picks and weights equal the CPU oracle's on that row.
 // Logits are published with cache-bypassing (sc1) stores; each block counts itself in once its
 // stores completed, and the last block loads the logits of all rows at once and
-// spreads the per-row work over its waves: for topk <= 8 and 2 B <= RT_WPB one wave selects
-// each row's top-k over all its experts (canon_select_topk) beside the B softmax
-// denominators; above 4 rows the 4 B group selections come first and one rank merge per row
-// replaces the row selection; the picks go out at once, then the weights follow; for topk > 8
-// one wave per row does both.  It writes idx, wts and sgate, and (tags != nullptr) also
+// spreads the per-row work over its waves: for topk <= 8 one wave selects each row's top-k over
+// all its experts (canon_select_topk) beside the B softmax denominators; the picks go out at once,
+// then the weights follow; for topk > 8 one wave per row does both.  It writes idx, wts and sgate, and (tags != nullptr) also
 // publishes them as tagged words
 // (tag << 32) | value bits with cache-bypassing stores, for blocks of the same launch to poll:
 // row r's experts at tags[r topk ..] (and, for B topk <= 32, in RR_REPS replicas), its
 // weights at tags[(B + r) topk ..], its shared-expert gate logit at tags[2 B topk + r].
-// It resets the counter.  Every thread returns normally (no early exit), so callers may add
-// work after it.
+// Blocks count themselves in by adding inc (1, or 65536 for a second set of rows on the same
+// word) and the last one takes its set's count off again.  Every thread returns normally (no early
+// exit), so callers may add work after it.
 #pragma once
 #include "canon.hpp"
 
@@ -36,8 +35,9 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
                            const float* __restrict__ nw, float eps, float* __restrict__ logits, int E, int topk,
                            int* __restrict__ idx, float* __restrict__ wts, float* __restrict__ sgate,
                            uint32_t* __restrict__ counter, uint64_t* __restrict__ tags, uint32_t tag,
-                           float4 (*xs)[2048 / 4]) {
+                           float4 (*xs)[2048 / 4], uint32_t inc = 1u) {
 #pragma clang fp contract(off)
+  static_assert(2 * B <= RT_WPB, "a selection and a denominator wave per row");
   constexpr int K = 2048, NCH = K / 8 / WAVE, NRM = K / 4 / WAVE, NT = RT_WPB * 64;
   __shared__ float s_inv[B];
   __shared__ int s_last;
@@ -93,11 +93,11 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0)
-    s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)nblk - 1;
+    s_last = (__hip_atomic_fetch_add(counter, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / inc & 0xffffu) ==
+             (uint32_t)nblk - 1;
   __syncthreads();
   if (!s_last) return;
   __shared__ float lg[B][257];
-  __shared__ uint64_t s_cand[B][32];
   __shared__ int s_sel[B][8];
   __shared__ float s_mz[B][2];
   {
@@ -131,27 +131,12 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
     }
   };
   if (topk <= 8) {
-    // the 4 B group selections first, then each row's rank merge (its picks are published at
-    // once: the gate_up blocks of the fused launch wait for them) beside the B softmax
-    // denominators, then the weights
-    constexpr bool kRowWave = 2 * B <= RT_WPB;  // one wave selects a whole row (8 rounds over 256)
-    if constexpr (!kRowWave) {
-      for (int t = wave; t < 4 * B; t += RT_WPB) {
-        int ck, ce;
-        canon_select_group8(lg[t >> 2], E, t & 3, &ck, &ce);
-        if (lane < 8) s_cand[t >> 2][(t & 3) * 8 + lane] = canon_cand64(ck, ce);
-      }
-      __syncthreads();
-    }
+    // each row's picks, published at once (the gate_up blocks of the fused launch wait for them), beside
+    // the B softmax denominators, then the weights
     for (int t = wave; t < 2 * B; t += RT_WPB) {
       if (t < B) {
-        int id;
-        if constexpr (kRowWave) {
-          id = canon_select_topk(lg[t], E, topk);
-          if (lane < topk) s_sel[t][lane] = id;
-        } else {
-          id = merge_picks(s_cand[t], s_sel[t], topk);
-        }
+        const int id = canon_select_topk(lg[t], E, topk);
+        if (lane < topk) s_sel[t][lane] = id;
         if (lane < topk) {
           idx[t * topk + lane] = id;
           if (tags) {
@@ -196,7 +181,7 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
       __hip_atomic_store(tags + 2 * B * topk + threadIdx.x, ((uint64_t)tag << 32) | __float_as_uint(lg[threadIdx.x][E]),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) __hip_atomic_fetch_sub(counter, inc * (uint32_t)nblk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace drm

@@ -277,3 +277,32 @@ def test_decode_rows_groups_match_calls_of_four(fmt, rows):
         torch.cuda.synchronize()
         out.append(bits(host(dx)))
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("rows,E,norm", [(5, 256, True), (6, 100, False), (7, 256, True), (8, 256, True), (8, 8, True)])
+def test_router_rows_two_sets_bit_exact(rows, E, norm):
+    """5 to 8 rows: two sets of router blocks on one counter word."""
+    test_router_rows_bit_exact_per_row(rows, E, norm)
+
+
+@pytest.mark.parametrize("rows", [2, 5, 8])
+def test_router_rows_more_than_eight_picks(rows):
+    """topk > 8 (one wave per row selects and weighs) in either set of rows."""
+    import torch
+
+    E, topk = 64, 12
+    L = synth.make_layer(290 + rows, E=E, fmt="cfg", quick=True)
+    x = np.random.default_rng(rows).normal(0, 1, (rows, H)).astype(np.float32)
+    t = {"w": dev(L["router"]), "x": dev(x), "nw": dev(L["nw"])}
+    logits, wts, sg = (torch.zeros(n, device="cuda") for n in (rows * (E + 1), rows * topk, rows))
+    idx, counter = (torch.zeros(n, dtype=torch.int32, device="cuda") for n in (rows * topk, 1))
+    P = D.ptr
+    D.lib().dr_router_topk_rows(P(t["w"]), P(t["x"]), P(t["nw"]), 1e-6, P(logits), E, topk, H, rows, P(idx), P(wts),
+                                P(sg), P(counter), D.stream_ptr())
+    torch.cuda.synchronize()
+    assert int(host(counter)[0]) == 0
+    for r in range(rows):
+        _, ri, rw, rs = O.router_topk(L["router"], x[r], L["nw"], 1e-6, E, topk)
+        np.testing.assert_array_equal(host(idx)[r * topk:(r + 1) * topk], ri)
+        np.testing.assert_array_equal(bits(host(wts)[r * topk:(r + 1) * topk]), bits(rw))
+        assert bits(host(sg)[r:r + 1])[0] == bits(np.float32(rs))
