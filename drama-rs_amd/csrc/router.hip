@@ -12,26 +12,25 @@ using namespace drm;
 
 namespace {
 
-// Decode router for B rows (B <= 4) in one launch of router blocks (router_rows.hpp).  With B2 > 0,
-// blockIdx.y = 1 is a second, independent router of the B2 rows after them, counted in the counter's upper
-// half: every block's time is its staging, norms and LDS reads per row, so 8 rows on twice the blocks
-// take 9 us where one set of blocks took 12.8 (4 rows: 8.3).
-template <int B, int B2>
+// Decode router of a few rows in one launch: sets of two rows (LAST in the last one), each with its own
+// router blocks (router_rows.hpp) and its own byte of the counter.  A block's time is its staging, norms
+// and LDS reads per row: 8 rows on one set of blocks took 12.8 us, on two sets 8.9, on four 8.1; 4 rows 8.6
+// on one set, 8.0 on two.
+template <int LAST>
 __global__ void __launch_bounds__(RT_WPB * 64)
     k_router_topk_rows(const uint16_t* __restrict__ W, const float* __restrict__ x, const float* __restrict__ nw,
                        float eps, float* __restrict__ logits, int E, int topk, int* __restrict__ idx,
                        float* __restrict__ wts, float* __restrict__ sgate, uint32_t* __restrict__ counter) {
-  __shared__ float4 xs[B][2048 / 4];
-  if constexpr (B2 > 0) {
-    static_assert(B2 <= B, "xs holds either set");
-    if (blockIdx.y == 1) {
-      router_rows_block<B2>(blockIdx.x, gridDim.x, W, x + (size_t)B * 2048, nw, eps, logits + (size_t)B * (E + 1), E,
-                            topk, idx + B * topk, wts + B * topk, sgate + B, counter, nullptr, 0u, xs, 65536u);
-      return;
-    }
-  }
-  router_rows_block<B>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr, 0u,
-                       xs);
+  __shared__ float4 xs[2][2048 / 4];
+  const int r = 2 * blockIdx.y;  // first row of the set
+  x += (size_t)r * 2048, logits += (size_t)r * (E + 1), idx += r * topk, wts += r * topk, sgate += r;
+  const uint32_t inc = 1u << (8 * blockIdx.y);
+  if (LAST == 2 || blockIdx.y + 1 < gridDim.y)
+    router_rows_block<2>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr, 0u,
+                         xs, inc);
+  else
+    router_rows_block<1>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr, 0u,
+                         xs, inc);
 }
 
 // One row per block.  topk <= 8: waves 0..3 each pick the top 8 of 64 experts and wave 4
@@ -289,7 +288,7 @@ API int dr_router_topk(const uint16_t* W, const float* x, const float* nw, float
   if (K != 2048 || E > 256 || E < 1 || topk > 32 || topk < 1 || topk > E) return -1;
   // the one-row case of the small-batch router (its one-wave top-k measured 0.3 us shorter per
   // call than four group selections and a rank merge, with the same picks)
-  hipLaunchKernelGGL((k_router_topk_rows<1, 0>), dim3((E + RT_WPB) / RT_WPB), dim3(RT_WPB * 64), 0, st, W, x, nw, eps, logits,
+  hipLaunchKernelGGL(k_router_topk_rows<1>, dim3((E + RT_WPB) / RT_WPB), dim3(RT_WPB * 64), 0, st, W, x, nw, eps, logits,
                      E, topk, idx, wts, sgate, counter);
   return 0;
 }
@@ -298,14 +297,10 @@ API int dr_router_topk_rows(const uint16_t* W, const float* x, const float* nw, 
                             int topk, int K, int rows, int* idx, float* wts, float* sgate, uint32_t* counter,
                             hipStream_t st) {
   if (K != 2048 || E > 256 || E < 1 || topk > 32 || topk < 1 || topk > E || rows < 1 || rows > 8) return -1;
-  const dim3 g((E + RT_WPB) / RT_WPB, rows > 4 ? 2 : 1), b(RT_WPB * 64);
-  switch (rows) {
-#define RT_ROWS(n) \
-  case n: hipLaunchKernelGGL((k_router_topk_rows<(n > 4 ? 4 : n), (n > 4 ? n - 4 : 0)>), g, b, 0, st, W, x, nw, eps, logits, \
-                             E, topk, idx, wts, sgate, counter); break;
-    RT_ROWS(1) RT_ROWS(2) RT_ROWS(3) RT_ROWS(4) RT_ROWS(5) RT_ROWS(6) RT_ROWS(7) RT_ROWS(8)
-#undef RT_ROWS
-  }
+  const dim3 g((E + RT_WPB) / RT_WPB, (rows + 1) / 2), b(RT_WPB * 64);
+  static_assert((256 + RT_WPB) / RT_WPB < 256, "a set's block count fits its byte of the counter");
+  auto kern = rows % 2 ? k_router_topk_rows<1> : k_router_topk_rows<2>;
+  hipLaunchKernelGGL(kern, g, b, 0, st, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter);
   return 0;
 }
 

@@ -17,8 +17,8 @@
 // (tag << 32) | value bits with cache-bypassing stores, for blocks of the same launch to poll:
 // row r's experts at tags[r topk ..] (and, for B topk <= 32, in RR_REPS replicas), its
 // weights at tags[(B + r) topk ..], its shared-expert gate logit at tags[2 B topk + r].
-// Blocks count themselves in by adding inc (1, or 65536 for a second set of rows on the same
-// word) and the last one takes its set's count off again.  Every thread returns normally (no early
+// Blocks count themselves in by adding inc (a byte of the counter word per set of rows: 1, 256, ..;
+// nblk < 256) and the last one takes its set's count off again.  Every thread returns normally (no early
 // exit), so callers may add work after it.
 #pragma once
 #include "canon.hpp"
@@ -93,7 +93,7 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0)
-    s_last = (__hip_atomic_fetch_add(counter, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / inc & 0xffffu) ==
+    s_last = (__hip_atomic_fetch_add(counter, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / inc & 0xffu) ==
              (uint32_t)nblk - 1;
   __syncthreads();
   if (!s_last) return;

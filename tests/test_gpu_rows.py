@@ -281,7 +281,7 @@ def test_decode_rows_groups_match_calls_of_four(fmt, rows):
 
 @pytest.mark.parametrize("rows,E,norm", [(5, 256, True), (6, 100, False), (7, 256, True), (8, 256, True), (8, 8, True)])
 def test_router_rows_two_sets_bit_exact(rows, E, norm):
-    """5 to 8 rows: two sets of router blocks on one counter word."""
+    """Sets of two rows, the last one full or not, on one counter word."""
     test_router_rows_bit_exact_per_row(rows, E, norm)
 
 
