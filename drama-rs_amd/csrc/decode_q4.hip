@@ -39,7 +39,8 @@ __global__ void __launch_bounds__(WPB * 64)
   static_assert(PPW * NW == B * DEC_TOPK * I && D <= PPW, "units split evenly over the routed waves");
   __shared__ float4 xs[B * H / 4];
   const int lane = lane_id(), wave = wave_id();
-  x += (size_t)blockIdx.y * B * H, idx += blockIdx.y * B * DEC_TOPK, act += (size_t)blockIdx.y * B * (DEC_TOPK + 1) * I;
+  if constexpr (B == 4)  // fewer rows are a single group
+    x += (size_t)blockIdx.y * B * H, idx += blockIdx.y * B * DEC_TOPK, act += (size_t)blockIdx.y * B * (DEC_TOPK + 1) * I;
   if ((int)blockIdx.x >= NBS) {
     const int g = (blockIdx.x - NBS) * WPB + wave;
     XStage<H, NT, B, SlotQ4D> xst;

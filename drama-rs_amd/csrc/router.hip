@@ -12,25 +12,27 @@ using namespace drm;
 
 namespace {
 
-// Decode router of a few rows in one launch: sets of two rows (LAST in the last one), each with its own
-// router blocks (router_rows.hpp) and its own byte of the counter.  A block's time is its staging, norms
+// Decode router of a few rows in one launch: sets of two rows (LAST in the last one; ONE: a single
+// set), each with its own router blocks (router_rows.hpp) and its own byte of the counter.  A block's time is its staging, norms
 // and LDS reads per row: 8 rows on one set of blocks took 12.8 us, on two sets 8.9, on four 8.1; 4 rows 8.6
 // on one set, 8.0 on two.
-template <int LAST>
+template <int LAST, bool ONE>
 __global__ void __launch_bounds__(RT_WPB * 64)
     k_router_topk_rows(const uint16_t* __restrict__ W, const float* __restrict__ x, const float* __restrict__ nw,
                        float eps, float* __restrict__ logits, int E, int topk, int* __restrict__ idx,
                        float* __restrict__ wts, float* __restrict__ sgate, uint32_t* __restrict__ counter) {
-  __shared__ float4 xs[2][2048 / 4];
-  const int r = 2 * blockIdx.y;  // first row of the set
+  __shared__ float4 xs[ONE ? LAST : 2][2048 / 4];
+  const int set = ONE ? 0 : blockIdx.y, r = 2 * set;  // r: first row of the set
   x += (size_t)r * 2048, logits += (size_t)r * (E + 1), idx += r * topk, wts += r * topk, sgate += r;
-  const uint32_t inc = 1u << (8 * blockIdx.y);
-  if (LAST == 2 || blockIdx.y + 1 < gridDim.y)
-    router_rows_block<2>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr, 0u,
-                         xs, inc);
-  else
-    router_rows_block<1>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr, 0u,
-                         xs, inc);
+  if constexpr (!ONE && LAST == 1) {
+    if (blockIdx.y + 1 < gridDim.y) {
+      router_rows_block<2, false>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter,
+                                  nullptr, 0u, xs, 8 * set);
+      return;
+    }
+  }
+  router_rows_block<LAST, ONE>(blockIdx.x, gridDim.x, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter, nullptr,
+                               0u, xs, 8 * set);
 }
 
 // One row per block.  topk <= 8: waves 0..3 each pick the top 8 of 64 experts and wave 4
@@ -288,7 +290,7 @@ API int dr_router_topk(const uint16_t* W, const float* x, const float* nw, float
   if (K != 2048 || E > 256 || E < 1 || topk > 32 || topk < 1 || topk > E) return -1;
   // the one-row case of the small-batch router (its one-wave top-k measured 0.3 us shorter per
   // call than four group selections and a rank merge, with the same picks)
-  hipLaunchKernelGGL(k_router_topk_rows<1>, dim3((E + RT_WPB) / RT_WPB), dim3(RT_WPB * 64), 0, st, W, x, nw, eps, logits,
+  hipLaunchKernelGGL((k_router_topk_rows<1, true>), dim3((E + RT_WPB) / RT_WPB), dim3(RT_WPB * 64), 0, st, W, x, nw, eps, logits,
                      E, topk, idx, wts, sgate, counter);
   return 0;
 }
@@ -299,7 +301,7 @@ API int dr_router_topk_rows(const uint16_t* W, const float* x, const float* nw, 
   if (K != 2048 || E > 256 || E < 1 || topk > 32 || topk < 1 || topk > E || rows < 1 || rows > 8) return -1;
   const dim3 g((E + RT_WPB) / RT_WPB, (rows + 1) / 2), b(RT_WPB * 64);
   static_assert((256 + RT_WPB) / RT_WPB < 256, "a set's block count fits its byte of the counter");
-  auto kern = rows % 2 ? k_router_topk_rows<1> : k_router_topk_rows<2>;
+  auto kern = rows == 1 ? k_router_topk_rows<1, true> : rows % 2 ? k_router_topk_rows<1, false> : k_router_topk_rows<2, false>;
   hipLaunchKernelGGL(kern, g, b, 0, st, W, x, nw, eps, logits, E, topk, idx, wts, sgate, counter);
   return 0;
 }

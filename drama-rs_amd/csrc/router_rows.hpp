@@ -17,9 +17,10 @@
 // (tag << 32) | value bits with cache-bypassing stores, for blocks of the same launch to poll:
 // row r's experts at tags[r topk ..] (and, for B topk <= 32, in RR_REPS replicas), its
 // weights at tags[(B + r) topk ..], its shared-expert gate logit at tags[2 B topk + r].
-// Blocks count themselves in by adding inc (a byte of the counter word per set of rows: 1, 256, ..;
-// nblk < 256) and the last one takes its set's count off again.  Every thread returns normally (no early
-// exit), so callers may add work after it.
+// Blocks count themselves in at bit shift of the counter word and the last one clears the count:
+// ALONE, the only set of rows on this counter, with a store of 0 (shift 0); otherwise each set has a
+// byte of the word (nblk < 256) and its last block takes the set's own count off again.  Every thread
+// returns normally (no early exit), so callers may add work after it.
 #pragma once
 #include "canon.hpp"
 
@@ -30,12 +31,12 @@ constexpr int RT_WPB = 8;  // router waves (= logit rows) per block
 // one replica per 256 bytes, B topk <= 32): hundreds of pollers on one cache line serialise.
 constexpr int RR_REPS = 16, RR_WORD0 = 128;
 
-template <int B>
+template <int B, bool ALONE = true>
 DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, const float* __restrict__ x,
                            const float* __restrict__ nw, float eps, float* __restrict__ logits, int E, int topk,
                            int* __restrict__ idx, float* __restrict__ wts, float* __restrict__ sgate,
                            uint32_t* __restrict__ counter, uint64_t* __restrict__ tags, uint32_t tag,
-                           float4 (*xs)[2048 / 4], uint32_t inc = 1u) {
+                           float4 (*xs)[2048 / 4], int shift = 0) {
 #pragma clang fp contract(off)
   static_assert(2 * B <= RT_WPB, "a selection and a denominator wave per row");
   constexpr int K = 2048, NCH = K / 8 / WAVE, NRM = K / 4 / WAVE, NT = RT_WPB * 64;
@@ -92,9 +93,10 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (threadIdx.x == 0)
-    s_last = (__hip_atomic_fetch_add(counter, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / inc & 0xffu) ==
-             (uint32_t)nblk - 1;
+  if (threadIdx.x == 0) {
+    const uint32_t n = __hip_atomic_fetch_add(counter, 1u << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = (ALONE ? n : n >> shift & 0xffu) == (uint32_t)nblk - 1;
+  }
   __syncthreads();
   if (!s_last) return;
   __shared__ float lg[B][257];
@@ -181,7 +183,12 @@ DEV void router_rows_block(int blk, int nblk, const uint16_t* __restrict__ W, co
       __hip_atomic_store(tags + 2 * B * topk + threadIdx.x, ((uint64_t)tag << 32) | __float_as_uint(lg[threadIdx.x][E]),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (threadIdx.x == 0) __hip_atomic_fetch_sub(counter, inc * (uint32_t)nblk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) {
+    if constexpr (ALONE)
+      __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+      __hip_atomic_fetch_sub(counter, (uint32_t)nblk << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 }  // namespace drm
