@@ -247,7 +247,8 @@ void launch_gate_up_b(const uint8_t* gu_q, const void* gu_sm, const int8_t* sgu_
 // rows independent decode rows (x, res, y: [rows, H]; idx, wts: [rows, topk]; act: rows x
 // (topk + 1) x I).  gate_up: the groups of 4 rows in one launch, the remaining 1 .. 3 rows in a second one;
 // down: one launch.  A pair of launches per 4 rows leaves the chip half idle at every boundary:
-// 20 rows (router included) 162 us that way, 108 now; 64 rows 504 -> 296.
+// 20 rows (three router calls included) 162 us that way, 108 with one launch, 97 with the router in sets of two rows; 64 rows
+// 504 -> 296 -> 259.
 template <class SC, class SH>
 int launch_decode(const uint8_t* gu_q, const void* gu_sm, const uint8_t* d_q, const void* d_sm, const int8_t* sgu_q,
                   const uint16_t* sgu_s, const int8_t* sd_q, const uint16_t* sd_s, const float* x, const int* idx,
