@@ -171,18 +171,19 @@ __global__ void __launch_bounds__(NW * 64)
 #pragma unroll
       for (int y = 0; y < BN; ++y) acc[s][x][y] = (f32x16)(0.f);
   uint4 av[D][S][BM], wv[D][S][BN];
-  // FULL: every chunk exists (K = 512 NCH); otherwise chunks past K / 8 are zero (fma(0, 0, sum) = sum)
-  auto chunk = [&](const uint16_t* row, int c) {
+  // FULL: every chunk exists (K = 512 NCH); otherwise chunks past K / 8 are -0 in A and +0 in W
+  // (fma(-0, +0, sum) = sum for every sum; a product of +0 would turn a sum of -0 into +0)
+  auto chunk = [&](const uint16_t* row, int c, uint32_t pad) {
     const uint4 v = ld16(row + (size_t)(FULL ? c : min(c, KC - 1)) * 8);
-    return FULL || c < KC ? v : make_uint4(0, 0, 0, 0);
+    return FULL || c < KC ? v : make_uint4(pad, pad, pad, pad);
   };
   auto load = [&](int j) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
 #pragma unroll
-      for (int x = 0; x < BM; ++x) av[j % D][s][x] = chunk(ap[x], c0 + 4 * s + 64 * j);
+      for (int x = 0; x < BM; ++x) av[j % D][s][x] = chunk(ap[x], c0 + 4 * s + 64 * j, 0x80008000u);
 #pragma unroll
-      for (int y = 0; y < BN; ++y) wv[j % D][s][y] = chunk(wp[y], c0 + 4 * s + 64 * j);
+      for (int y = 0; y < BN; ++y) wv[j % D][s][y] = chunk(wp[y], c0 + 4 * s + 64 * j, 0u);
     }
   };
 #pragma unroll

@@ -219,3 +219,23 @@ def test_gemm_matrix_unit_bit_exact(M, N, K, beta):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     np.testing.assert_array_equal(bits(got[ok]), bits(want[ok]))
+
+
+@pytest.mark.parametrize("M,N,K", [(6, 40, 520), (40, 300, 1000), (300, 257, 1496), (520, 513, 3000), (6, 40, 2048)])
+def test_gemm_negative_zero_sums(M, N, K):
+    """Products below the subnormals, all negative: every canonical lane sum is -0 and so is every dot, also
+    where some lanes have one chunk fewer than others."""
+    import torch
+
+    A, Wt = (synth.f32_to_bf16(np.full((n, K), v, np.float32)) for n, v in ((M, 1e-30), (N, -1e-30)))
+    ref = np.asarray(O.router_logits_rows(A[:1], Wt[:1], 1, 1, K), np.float32)
+    assert bits(ref)[0] == 0x80000000
+    C = torch.ones(M, N, device="cuda")
+    h = np.zeros(1, np.uint64)
+    L = D.lib()
+    L.dr_cublas_create(h.ctypes.data, D.stream_ptr())
+    dA, dWt = dev(A), dev(Wt)
+    L.dr_gemm(int(h[0]), D.ptr(dA), D.ptr(dWt), D.ptr(C), M, N, K, 0.0)
+    torch.cuda.synchronize()
+    L.dr_cublas_destroy(int(h[0]))
+    np.testing.assert_array_equal(bits(host(C)), np.full(M * N, 0x80000000, np.uint32).reshape(bits(host(C)).shape))
