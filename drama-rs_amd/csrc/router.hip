@@ -130,6 +130,9 @@ __global__ void __launch_bounds__(512)
   }
 }
 
+// one chunk of -0 and one of +0 (k_gemm_mfma)
+__device__ const uint4 k_pad[2] = {{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u}, {0u, 0u, 0u, 0u}};
+
 // The same canonical GEMM on the fp32 matrix unit.  v_mfma_f32_16x16x1_4b_f32 is four independent 16 x 16
 // rank-1 updates whose every element is one fp32 fma (rounded to nearest even, subnormals kept, checked
 // against fmaf), so block b of an instruction can carry the running sum of one canonical lane: set s
@@ -140,13 +143,15 @@ __global__ void __launch_bounds__(512)
 // sets, then over the NW waves through LDS (a + b = b + a, so the same bits as the butterfly).
 // The matrix unit does 32 of these fmas per clock and SIMD where the vector unit does 16, and
 // the bf16 -> fp32 conversions fall from one per 8 / 5 fmas to one per 16 and matrix row.
-// Block: 16 BM x 16 BN outputs, NW waves of 64 / NW canonical lanes each.  Consecutive tiles of
+// Block: 16 BM x 16 BN outputs, NW waves of 64 / NW canonical lanes each, four waves per SIMD (at most 128
+// registers: two blocks of 8 waves per CU).  Consecutive tiles of
 // one XCD share their W rows.
 // What bounds it: large shapes the loads (16 rows x 64 bytes per instruction, ~8 TB/s of L2 reads; 32 x 32
-// tiles run at 65% of the fp32 matrix rate), small ones the 2048-long chains of one tile (7 us per 32 x 32).
+// tiles run at 65% of the fp32 matrix rate), small ones the MFMAs of one tile (K = 2048, 32 x 32: 128 per wave, four
+// waves per SIMD, 33 clocks each: 7 us).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 template <int NCH, int BM, int BN, int NW, bool FULL>
-__global__ void __launch_bounds__(NW * 64)
+__global__ void __launch_bounds__(NW * 64, 4)
     k_gemm_mfma(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, float* __restrict__ C, int M, int N,
                 int K, float beta) {
   constexpr int S = 16 / NW;               // sets of four canonical lanes per wave
@@ -172,25 +177,35 @@ __global__ void __launch_bounds__(NW * 64)
       for (int y = 0; y < BN; ++y) acc[s][x][y] = (f32x16)(0.f);
   uint4 av[D][S][BM], wv[D][S][BN];
   // FULL: every chunk exists (K = 512 NCH); otherwise chunks past K / 8 are -0 in A and +0 in W
-  // (fma(-0, +0, sum) = sum for every sum; a product of +0 would turn a sum of -0 into +0)
-  auto chunk = [&](const uint16_t* row, int c, uint32_t pad) {
-    const uint4 v = ld16(row + (size_t)(FULL ? c : min(c, KC - 1)) * 8);
-    return FULL || c < KC ? v : make_uint4(pad, pad, pad, pad);
+  // (fma(-0, +0, sum) = sum for every sum; a product of +0 would turn a sum of -0 into +0).  With more than one
+  // round they are loaded from k_pad: a select on the loaded words would wait for them where they are requested
+  auto chunk = [&](const uint16_t* row, int c, int pad) {
+    const uint16_t* p = row + (size_t)c * 8;
+    if (FULL) return ld16(p);
+    if (NCH > 1) return ld16(c < KC ? p : reinterpret_cast<const uint16_t*>(k_pad + pad));
+    const uint32_t z = pad == 0 ? 0x80008000u : 0u;
+    const uint4 v = ld16(row + (size_t)min(c, KC - 1) * 8);
+    return c < KC ? v : make_uint4(z, z, z, z);
   };
+  // round j has a chunk: without asking up to NCH / 2, since K > 256 NCH for NCH > 1 (NCH = 8: asked from the
+  // second round on, which keeps the unrolled rounds apart and the 8-wave tile at 125 registers, not 136)
+  auto round_in = [&](int j) { return FULL || j <= (NCH < 8 ? NCH / 2 : 0) || 64 * j < KC; };
   auto load = [&](int j) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
 #pragma unroll
-      for (int x = 0; x < BM; ++x) av[j % D][s][x] = chunk(ap[x], c0 + 4 * s + 64 * j, 0x80008000u);
+      for (int x = 0; x < BM; ++x) av[j % D][s][x] = chunk(ap[x], c0 + 4 * s + 64 * j, 0);
 #pragma unroll
-      for (int y = 0; y < BN; ++y) wv[j % D][s][y] = chunk(wp[y], c0 + 4 * s + 64 * j, 0u);
+      for (int y = 0; y < BN; ++y) wv[j % D][s][y] = chunk(wp[y], c0 + 4 * s + 64 * j, 1);
     }
   };
 #pragma unroll
-  for (int j = 0; j < D; ++j) load(j);
+  for (int j = 0; j < D; ++j)
+    if (round_in(j)) load(j);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
+    if (!round_in(j)) break;
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
@@ -210,7 +225,7 @@ __global__ void __launch_bounds__(NW * 64)
           for (int y = 0; y < BN; ++y)
             acc[s][x][y] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[x], w[y], acc[s][x][y], 0, 0, 0);
       }
-    if (j + D < NCH) load(j + D);
+    if (j + D < NCH && round_in(j + D)) load(j + D);
     __builtin_amdgcn_sched_barrier(0);
   }
   // D layout: register 4 b + r of lane l is row 4 (l / 16) + r, column l % 16 of block b
@@ -253,10 +268,15 @@ template <int NCH, int BM, int BN, int NW>
 void launch_gemm_mfma(const uint16_t* A, const uint16_t* W, float* C, int M, int N, int K, float beta, hipStream_t st) {
   const int tiles = ((M + 16 * BM - 1) / (16 * BM)) * ((N + 16 * BN - 1) / (16 * BN));
   const dim3 grid((tiles + 7) / 8 * 8), block(NW * 64);
-  if (K == NCH * 512)
-    hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, true>), grid, block, 0, st, A, W, C, M, N, K, beta);
-  else
-    hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, false>), grid, block, 0, st, A, W, C, M, N, K, beta);
+  // K = 4096, 8 waves: always the instance with chunk bounds, since the other would need 135 registers
+  // (one block per CU: 300 x 1024 x 4096 40.6 us against 38.1, 1024 x 1024 108 against 97)
+  if constexpr (NW != 8 || NCH != 8) {
+    if (K == NCH * 512) {
+      hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, true>), grid, block, 0, st, A, W, C, M, N, K, beta);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, false>), grid, block, 0, st, A, W, C, M, N, K, beta);
 }
 
 // The largest tile whose blocks still fit the 256 CUs at once (a block's time is its tile's), us at K = 2048

@@ -239,3 +239,14 @@ def test_gemm_negative_zero_sums(M, N, K):
     torch.cuda.synchronize()
     L.dr_cublas_destroy(int(h[0]))
     np.testing.assert_array_equal(bits(host(C)), np.full(M * N, 0x80000000, np.uint32).reshape(bits(host(C)).shape))
+
+
+@pytest.mark.parametrize("K", [504, 512, 1000, 1024, 1496, 2048, 3000, 4096])
+@pytest.mark.parametrize("M,N", [
+    (5, 33), (17, 2049),   # 16 x 16 and 32 x 16 tiles
+    (17, 4104),            # 32 x 32 tiles
+    (100, 3000),           # 32 x 16 tiles, 8 waves
+])
+def test_gemm_every_tile_bit_exact(M, N, K):
+    """Every tile with every number of chunk rounds, all of them full or the last ones short."""
+    test_gemm_matrix_unit_bit_exact(M, N, K, 0.0)
