@@ -6,6 +6,8 @@
 // hence the selected experts bit for bit.
 #include "router_rows.hpp"
 
+#include <algorithm>
+
 #pragma clang fp contract(off)
 
 using namespace drm;
@@ -279,26 +281,34 @@ void launch_gemm_mfma(const uint16_t* A, const uint16_t* W, float* C, int M, int
   hipLaunchKernelGGL((k_gemm_mfma<NCH, BM, BN, NW, false>), grid, block, 0, st, A, W, C, M, N, K, beta);
 }
 
-// The largest tile whose blocks still fit the 256 CUs at once (a block's time is its tile's), us at K = 2048
-// for 16 x 16, 32 x 16 (16 waves), 32 x 32 tiles: 100 x 257 5.8 / 8.1 / 12.0, 300 x 257 9.6 / 8.6 / 12.3,
-// 512 x 257 13.6 / 15.3 / 12.6.  Past one round of 32 x 32 tiles, two 8-wave blocks of 32 x 16 per CU
-// (1024 x 257 24.4 -> 21.2, 300 x 1024 24.1 -> 21.3; K = 512: 300 x 2048 13.2 -> 11.7) until a second round of 32 x 32
-// tiles is well filled (512 x 1024 28.0 -> 25.1).  The vector kernel this replaces (8 x 5 outputs per wave):
-// 6.9 us at 100 x 257, 8.5 at 300, 15.3 at 512, 28.0 at 1024, 49.7 at 512 x 1024, 26.4 at 512 x 2048 x 512.
+// The tile with the least cost a + b r, r the rounds of 256 tiles: fitted to the times of every tile over 5 to
+// 1024 rows, 33 to 16384 columns and K = 504 to 4096 (units of 10 ns at K = 2048, where the order is that of every
+// larger K, and at K = 512).  Few tiles: the smallest, whose waves have the fewest products; many: the large
+// ones, which load less per product, as long as their last round and their rows past M cost less than that saves.
+// us at K = 2048 for 16 x 16, 32 x 16 or 16 x 32, 32 x 32, 32 x 16 tiles of 8 waves: 100 x 257 5.8 / 8.1 / 12.0 / 8.7,
+// 300 x 257 9.4 / 8.1 / 12.2 / 8.8, 512 x 257 13.0 / 14.6 / 12.2 / 14.3, 1024 x 257 20.0 / 21 / 23.5 / 19.9, 5 x 4104 7.3 /
+// 7.6 (16 x 32) / 11.2 / 12.3.  The vector kernel this replaces: 6.9, 8.5, 15.3, 28.0 and 9.5; it was the faster one (by up
+// to 15%, K <= 1024) only where 17 to 32 rows meet a little over 4096 columns: 257 tiles or more at every size but 32 x 32.
 template <int NCH>
 void launch_gemm(const uint16_t* A, const uint16_t* W, float* C, int M, int N, int K, float beta, hipStream_t st) {
-  constexpr long long CUS = 256;
-  const long long m16 = (M + 15ll) / 16, m32 = (M + 31ll) / 32, n16 = (N + 15ll) / 16, n32 = (N + 31ll) / 32;
-  if (M <= GR_MAXM)
+  if (M <= GR_MAXM) {
     hipLaunchKernelGGL(k_gemm_rows<NCH>, dim3((N + 7) / 8), dim3(512), 0, st, A, W, C, M, N, K, beta);
-  else if (m16 * n16 <= CUS)
-    launch_gemm_mfma<NCH, 1, 1, 16>(A, W, C, M, N, K, beta, st);
-  else if (m32 * n16 <= CUS)
-    launch_gemm_mfma<NCH, 2, 1, 16>(A, W, C, M, N, K, beta, st);
-  else if (m32 * n32 <= CUS || (K > 512 && 2 * m32 * n32 > 3 * CUS))
-    launch_gemm_mfma<NCH, 2, 2, 16>(A, W, C, M, N, K, beta, st);
-  else
-    launch_gemm_mfma<NCH, 2, 1, 8>(A, W, C, M, N, K, beta, st);
+    return;
+  }
+  const long long m16 = (M + 15ll) / 16, m32 = (M + 31ll) / 32, n16 = (N + 15ll) / 16, n32 = (N + 31ll) / 32;
+  auto cost = [](long long tiles, int a1, int b1, int a, int b) {
+    const long long r = (tiles + 255) / 256;
+    return NCH == 1 ? a1 + b1 * r : a + b * r;
+  };
+  const long long c11 = cost(m16 * n16, 240, 120, 230, 350), c21 = cost(m32 * n16, 200, 175, 150, 655);
+  const long long c12 = cost(m16 * n32, 200, 176, 150, 660), c22 = cost(m32 * n32, 100, 390, 90, 1120);
+  const long long c8 = cost(m32 * n16, 220, 164, 330, 550);
+  const long long c = std::min({c11, c21, c12, c22, c8});
+  if (c == c11) launch_gemm_mfma<NCH, 1, 1, 16>(A, W, C, M, N, K, beta, st);
+  else if (c == c21) launch_gemm_mfma<NCH, 2, 1, 16>(A, W, C, M, N, K, beta, st);
+  else if (c == c12) launch_gemm_mfma<NCH, 1, 2, 16>(A, W, C, M, N, K, beta, st);
+  else if (c == c22) launch_gemm_mfma<NCH, 2, 2, 16>(A, W, C, M, N, K, beta, st);
+  else launch_gemm_mfma<NCH, 2, 1, 8>(A, W, C, M, N, K, beta, st);
 }
 
 }  // namespace

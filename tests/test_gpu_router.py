@@ -243,9 +243,11 @@ def test_gemm_negative_zero_sums(M, N, K):
 
 @pytest.mark.parametrize("K", [504, 512, 1000, 1024, 1496, 2048, 3000, 4096])
 @pytest.mark.parametrize("M,N", [
-    (5, 33), (17, 2049),   # 16 x 16 and 32 x 16 tiles
+    (5, 33), (100, 3000),  # 16 x 16 tiles; 32 x 16 tiles, 8 waves (K > 512)
+    (17, 2049),            # 32 x 16 tiles, 16 waves
+    (5, 4104),             # a row tile that is mostly empty
     (17, 4104),            # 32 x 32 tiles
-    (100, 3000),           # 32 x 16 tiles, 8 waves
+    (17, 9001),            # 32 x 16 tiles, 8 waves (K <= 512)
 ])
 def test_gemm_every_tile_bit_exact(M, N, K):
     """Every tile with every number of chunk rounds, all of them full or the last ones short."""
