@@ -1372,12 +1372,21 @@ inline int resident_blocks(const void* kern, int threads, size_t lds) {
 }
 
 // k_grouped_pass from 14 top-8 picks per expert on (448 token rows at 256 experts), where experts with a
-// second 16-token pass become common.  Whole prefill layers at 256 experts, k_grouped ->
+// second 16-token pass become common, and only from enough rows on that its items (twice the rows and tokens of
+// k_grouped's) fill the 256 blocks several times: 448 rows (int4), 384 (fp8, tile-step copy), 256 (fp8,
+// reference layout).  Whole prefill layers at 256 experts, k_grouped ->
 // k_grouped_pass: int4 300 rows 147 -> 150 us, 449 rows 173 -> 174, 512 (reference layout) 201 -> 194, 1024
 // 303 -> 264, hot experts 460 / 900 rows 170 / 249 -> 160 / 223; fp8 12 rows 94 -> 104, 300 rows 203 -> 207,
-// 460 rows 226 -> 227, 600 rows 258 -> 243.  The number of rows is only known where they come through
-// a row map; elsewhere (x_rows 0) k_grouped stays.
-inline bool use_passes(int x_rows, int E) { return (long long)x_rows * 8 >= 14ll * E; }
+// 460 rows 226 -> 227, 600 rows 258 -> 243.  Fewer experts, gate_up and down alone, time over k_grouped's at the 14
+// picks: int4 144 / 112 / 96 / 72 / 48 / 24 experts 1.12 / 1.08 / 1.18 / 1.34 / 1.67 / 2.3 (hot experts still 1.09 at 352
+// rows of 128), fp8 1.06 / 0.98 / 1.00 / 1.20 / 1.39 / 1.96, its copy 1.07 / 1.01 / 1.01 / 1.22 / 1.20 / 1.69; from the rows
+// above on 0.75 to 1.05 everywhere.  The number of rows is only known where they come through
+// a row map; elsewhere (x_rows 0) k_grouped stays.  The number of picks is not known at all: at 2 picks per row
+// the kernel chosen from 448 rows and 256 experts on takes 3 to 11% longer than k_grouped would.
+template <class F>
+inline bool use_passes(int x_rows, int E, bool packed) {
+  return x_rows >= (F::paired ? 448 : packed ? 384 : 256) && (long long)x_rows * 8 >= 14ll * E;
+}
 
 template <class F>
 void launch_grouped(const uint8_t* wq, const void* ws, const uint16_t* X, const int* offsets, const int* counts,
@@ -1401,7 +1410,7 @@ void launch_grouped(const uint8_t* wq, const void* ws, const uint16_t* X, const 
     // grouped experts: a persistent grid of as many blocks as are resident at once, walking the
     // work items (expert, token pass, row block) the kernel derives from counts
     const dim3 block(PF_GWPB * 64);
-    if (use_passes(x_rows, E)) {
+    if (use_passes<F>(x_rows, E, packed)) {
       auto kern = packed ? (mode == 1 ? k_grouped_pass<F, 1, 512, false, true>
                                       : rmap ? k_grouped_pass<F, 0, 2048, true, true> : k_grouped_pass<F, 0, 2048, false, true>)
                          : (mode == 1 ? k_grouped_pass<F, 1, 512, false, false>

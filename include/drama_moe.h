@@ -205,7 +205,8 @@ int dr_moe_group_rows(const int* idx, int rows, int topk, int e, int* counts, in
 /* dr_moe_prefill with the gate_up inputs read straight from the x_rows token rows of x through
  * row_of_slot (from dr_moe_topk_group) instead of from a gathered xp: the same act and y bits as
  * dr_moe_gather_rows followed by dr_moe_prefill, one launch and the xp copy fewer.  Formats as
- * dr_moe_prefill, dr_moe_prefill_bf16s, dr_moe_prefill_fp8 and dr_moe_prefill_fp8_bf16s. */
+ * dr_moe_prefill, dr_moe_prefill_bf16s, dr_moe_prefill_fp8 and dr_moe_prefill_fp8_bf16s.  Which of
+ * two kernels runs (the same bits) goes by x_rows and e and presumes 8 picks per row. */
 int dr_moe_prefill_rows(const uint8_t* gu_q, const dr_half* gu_sm, const uint8_t* d_q, const dr_half* d_sm,
                         const dr_bf16* x, int x_rows, const int* row_of_slot, const int* offsets, const int* counts,
                         dr_bf16* act, float* y, int e, int h, int i, dr_stream_t st);

@@ -664,3 +664,59 @@ def test_prefill_passes_match_tiles(kind, fmt, packed, counts):
     assert lib.dr_last_error() == 0
     assert outs[0][1].any()
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("kind,fmt,packed", [("q4", "ref", True), ("q4", "cfg", False), ("fp8", "ref", False),
+                                             ("fp8", "cfg", True)])
+@pytest.mark.parametrize("counts", [[0] * 9, [14] + [0] * 8, [3, 0, 0, 40, 0, 1, 0, 16, 5]])
+def test_prefill_passes_few_tokens(kind, fmt, packed, counts):
+    """The kernel of the larger token counts with fewer items than blocks, or none, and infinities and NaN in some
+    token rows: the bits of the other kernel, finite values for finite rows, nothing written past the tokens."""
+    import torch
+
+    E, n, rows = len(counts), sum(counts), 448
+    lib, P, st = D.lib(), D.ptr, D.stream_ptr()
+    g = torch.Generator(device="cuda").manual_seed(n + E)
+    L = {k: dev(v) for k, v in synth.make_layer(47, E=E, fmt=fmt, kind=kind, quick=True).items()
+         if k in ("gu_q", "gu_s", "d_q", "d_s")}
+    W = dict(L)
+    if packed:
+        for q, s, nn, kk in (("gu_q", "gu_s", 2 * I, H), ("d_q", "d_s", H, I)):
+            W[q] = torch.zeros_like(L[q])
+            if kind == "q4":
+                W[s] = torch.zeros_like(L[s])
+                lib.dr_moe_pack_q4(P(L[q]), P(L[s]), E, nn, kk, P(W[q]), P(W[s]), st)
+            else:
+                lib.dr_moe_pack_fp8(P(L[q]), E, nn, kk, P(W[q]), st)
+    x = torch.randn(rows, H, generator=g, device="cuda").to(torch.bfloat16)
+    ros = torch.randint(3, rows, (n + 16,), generator=g, device="cuda", dtype=torch.int32)
+    for r, v in enumerate((float("inf"), float("nan"), -float("inf"))):
+        x[r, 100 * r + 7] = v
+        if n:
+            ros[5 * r + 1] = r
+    cnt = torch.tensor(counts, dtype=torch.int32, device="cuda")
+    off = (torch.cumsum(cnt, 0) - cnt).to(torch.int32)
+    sfx = ("_fp8" if kind == "fp8" else "") + ("_bf16s" if fmt == "cfg" else "")
+    outs = []
+    for passes in (True, False):
+        act = torch.full((n + 4, I), 77, dtype=torch.int16, device="cuda")
+        y = torch.full((n + 4, H), 7.0, device="cuda")
+        if passes:
+            getattr(lib, "dr_moe_prefill_rows" + ("_packed" if packed else "") + sfx)(
+                P(W["gu_q"]), P(W["gu_s"]), P(W["d_q"]), P(W["d_s"]), P(x), rows, P(ros), P(off), P(cnt), P(act), P(y),
+                E, H, I, st)
+        else:
+            xp = x[ros.long()].contiguous()
+            getattr(lib, "dr_moe_prefill" + sfx)(P(L["gu_q"]), P(L["gu_s"]), P(L["d_q"]), P(L["d_s"]), P(xp), P(off),
+                                                 P(cnt), P(act), P(y), E, H, I, st)
+        torch.cuda.synchronize()
+        outs.append((act, y))
+    (a0, y0), (a1, y1) = outs
+    assert lib.dr_last_error() == 0
+    assert (a0[n:] == 77).all() and (y0[n:] == 7.0).all()
+    if n:
+        finite = (ros[:n] > 2)
+        assert y0[:n][finite].isfinite().all() and not y0[:n][~finite].isfinite().all()
+    for p, q in ((a0.view(torch.bfloat16), a1.view(torch.bfloat16)), (y0, y1)):
+        assert torch.equal(p.isnan(), q.isnan())
+        assert torch.equal(p.nan_to_num(nan=0.0).view(p.dtype), q.nan_to_num(nan=0.0).view(p.dtype))
