@@ -988,7 +988,11 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
       if (16 * t >= it.ntok) break;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int row = (16 * t + 4 * g + i) * NO + it.n0;
+        int row = (16 * t + 4 * g + i) * NO;
+        // fp8: the last of these offsets stays out of the registers kept across the steps (one instance had spilled
+        // a register for it; the times are the same either way).  All of them out: 1 to 2% slower
+        if (MODE == 0 && !F::paired && t == PASS / 16 - 1 && i == 3) asm volatile("" : "+v"(row));
+        row += it.n0;
         if constexpr (MODE == 0) {
           __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(silu(acc[0][t][i]) * acc[1][t][i]), rs, (row + c16) * OB, 0, 0);
         } else {
@@ -1380,7 +1384,7 @@ inline int resident_blocks(const void* kern, int threads, size_t lds) {
 // 460 rows 226 -> 227, 600 rows 258 -> 243.  Fewer experts, gate_up and down alone, time over k_grouped's at the 14
 // picks: int4 144 / 112 / 96 / 72 / 48 / 24 experts 1.12 / 1.08 / 1.18 / 1.34 / 1.67 / 2.3 (hot experts still 1.09 at 352
 // rows of 128), fp8 1.06 / 0.98 / 1.00 / 1.20 / 1.39 / 1.96, its copy 1.07 / 1.01 / 1.01 / 1.22 / 1.20 / 1.69; from the rows
-// above on 0.75 to 1.05 everywhere.  The number of rows is only known where they come through
+// above on 0.75 to 1.05 (int4) and 0.50 to 1.05 (fp8).  The number of rows is only known where they come through
 // a row map; elsewhere (x_rows 0) k_grouped stays.  The number of picks is not known at all: at 2 picks per row
 // the kernel chosen from 448 rows and 256 experts on takes 3 to 11% longer than k_grouped would.
 template <class F>
