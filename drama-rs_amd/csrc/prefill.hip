@@ -53,19 +53,13 @@ DEV f32x4 mfma(const uint4& a, const uint4& b, const f32x4& c) {
 template <class SC>
 struct FmtQ4 {
   static constexpr bool q8 = false;
-  static constexpr bool has_min = true;
   static constexpr bool paired = true;  // k_grouped: 16-byte loads covering two groups per row
-  static constexpr bool packable = true;  // has a tile-step layout (dr_moe_pack_q4)
-  static constexpr int scale_group = 64;  // inputs per scale
   static DEV size_t row_bytes(int K) { return (size_t)K / 2; }
-  // fragment bytes of (row, group G) for lane group g: 8 bytes = 16 nibbles
-  static DEV void load(const uint8_t* row, int G, int g, uint2& raw) { raw = ld8(row + G * 32 + g * 8); }
   // (scale, min) of row n, group G: raw word, then decoded
   static DEV uint32_t scale_raw(const void* S, size_t n, int G, int K) {
     return reinterpret_cast<const uint32_t*>(S)[n * (K / 64) + G];
   }
   static DEV float2 scale_val(uint32_t w) { return SC::pair(w); }
-  static DEV float2 scale(const void* S, size_t n, int G, int K) { return scale_val(scale_raw(S, n, G, K)); }
 };
 
 // int8 (fragments in the order 0 4 1 5 2 6 3 7): 16 bytes per lane and group; bytes k..k+15 of the group slice, reordered
@@ -73,9 +67,7 @@ template <class SH>
 struct FmtQ8 {
   using Scale = SH;
   static constexpr bool q8 = true;
-  static constexpr bool has_min = false;
   static constexpr bool paired = false;
-  static constexpr bool packable = false;
   static constexpr int scale_group = SH::per_row ? 0 : 128;
   static DEV size_t row_bytes(int K) { return (size_t)K; }
   static DEV void load(const uint8_t* row, int G, int g, uint4& raw) { raw = ld16(row + G * 64 + g * 16); }
@@ -102,10 +94,7 @@ struct FmtQ8 {
 template <int SF>
 struct FmtFP8 {
   static constexpr bool q8 = false;
-  static constexpr bool has_min = false;
   static constexpr bool paired = false;
-  static constexpr bool packable = true;  // has a tile-step layout (dr_moe_pack_fp8)
-  static constexpr int scale_group = 128;
   static DEV size_t row_bytes(int K) { return (size_t)K; }
   static DEV void load(const uint8_t* row, int G, int g, uint4& raw) { raw = ld16(row + G * 64 + g * 16); }
   // 16 e4m3 bytes -> two bf16 fragments in input order (exact: every e4m3 value is a bf16 value)
@@ -123,15 +112,10 @@ struct FmtFP8 {
     return SF ? (uint32_t)reinterpret_cast<const uint16_t*>(S)[i] << 16 : reinterpret_cast<const uint32_t*>(S)[i];
   }
   static DEV float2 scale_val(uint32_t w) { return make_float2(__uint_as_float(w), 0.f); }
-  static DEV float2 scale(const void* S, size_t n, int G, int K) { return scale_val(scale_raw(S, n, G, K)); }
 };
 
 template <class F>
 struct Raw;
-template <class SC>
-struct Raw<FmtQ4<SC>> {
-  using T = uint2;
-};
 template <class SH>
 struct Raw<FmtQ8<SH>> {
   using T = uint4;
@@ -431,7 +415,6 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
     } else if constexpr (PK) {
       // fp8 block (tile n / 16, step): 1024 bytes per group, lane l's 16 bytes of group i at
       // i 1024 + 16 l (the block scales keep their layout)
-      static_assert(F::packable, "no tile-step layout for this format");
       const size_t blk = (n >> 4) * SPT + (size_t)(s % SPT);
       const uint8_t* tb = it.wq + blk * 4096;
       const int G0 = (s % SPT) * 4;
@@ -1141,7 +1124,6 @@ __global__ void __launch_bounds__(PF_WPB * 64)
   const char* ws = reinterpret_cast<const char*>(Ws) + (size_t)e * expert_s_elems * s_elem_bytes;
   const size_t rb = F::row_bytes(K);
   const int G0 = wave * GPW;
-  const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
   const f32x4 z = {0.f, 0.f, 0.f, 0.f};
   Wts<F> cur[GPW];
   load_tile<F, MODE, K>(wq, ws, rb, half, blockIdx.y * 16, G0, g, c16, cur);
@@ -1194,26 +1176,16 @@ __global__ void __launch_bounds__(PF_WPB * 64)
           }
         } else {
           const f32x4 accA = mfma(x1[i], a1, mfma(x0[i], a0, z));
-          f32x4 xg = z;
-          if (F::has_min) xg = mfma(x1[i], ones, mfma(x0[i], ones, z));
-          const float2 pa = F::scale_val(cur[i].sa);
-          const float ca = pa.y - 128.f * pa.x;
+          const float pa = F::scale_val(cur[i].sa).x;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            tA[r] = __builtin_fmaf(pa.x, accA[r], tA[r]);
-            if (F::has_min) tA[r] = __builtin_fmaf(ca, xg[r], tA[r]);
-          }
+          for (int r = 0; r < 4; ++r) tA[r] = __builtin_fmaf(pa, accA[r], tA[r]);
           if (MODE == 0) {
             uint4 b0, b1;
             F::convert(cur[i].b, b0, b1);
             const f32x4 accB = mfma(x1[i], b1, mfma(x0[i], b0, z));
-            const float2 pb = F::scale_val(cur[i].sb);
-            const float cb = pb.y - 128.f * pb.x;
+            const float pb = F::scale_val(cur[i].sb).x;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              tB[r] = __builtin_fmaf(pb.x, accB[r], tB[r]);
-              if (F::has_min) tB[r] = __builtin_fmaf(cb, xg[r], tB[r]);
-            }
+            for (int r = 0; r < 4; ++r) tB[r] = __builtin_fmaf(pb, accB[r], tB[r]);
           }
         }
       }
@@ -1415,18 +1387,15 @@ void launch_grouped(const uint8_t* wq, const void* ws, const uint16_t* X, const 
     // work items (expert, token pass, row block) the kernel derives from counts
     const dim3 block(PF_GWPB * 64);
     if (use_passes<F>(x_rows, E, packed)) {
-      auto kern = packed ? (mode == 1 ? k_grouped_pass<F, 1, 512, false, true>
-                                      : rmap ? k_grouped_pass<F, 0, 2048, true, true> : k_grouped_pass<F, 0, 2048, false, true>)
-                         : (mode == 1 ? k_grouped_pass<F, 1, 512, false, false>
-                                      : rmap ? k_grouped_pass<F, 0, 2048, true, false> : k_grouped_pass<F, 0, 2048, false, false>);
+      auto kern = packed ? (mode == 1 ? k_grouped_pass<F, 1, 512, false, true> : k_grouped_pass<F, 0, 2048, true, true>)
+                         : (mode == 1 ? k_grouped_pass<F, 1, 512, false, false> : k_grouped_pass<F, 0, 2048, true, false>);
       hipLaunchKernelGGL(kern, dim3(resident_blocks((const void*)kern, PF_GWPB * 64, 0)), block, 0, st, wq, ws, X,
                          offsets, counts, out, N, eq, es, sb, E, rmap, x_rows);
       return;
     }
     const size_t lds = 2 * ((size_t)PF_TOK * K * 2 + (F::paired ? (size_t)(K / 64) * PF_TOK * 4 : 0)) + 192 * 16 +
                        (mode == 0 ? 2 * PF_GRPW * (PF_GWPB / 2) * 64 * 16 : 0);
-    auto kern = packed ? (mode == 1 ? k_grouped<F, 1, 512, false, true>
-                                    : rmap ? k_grouped<F, 0, 2048, true, true> : k_grouped<F, 0, 2048, false, true>)
+    auto kern = packed ? (mode == 1 ? k_grouped<F, 1, 512, false, true> : k_grouped<F, 0, 2048, true, true>)
                        : (mode == 1 ? k_grouped<F, 1, 512, false, false>
                                     : rmap ? k_grouped<F, 0, 2048, true, false> : k_grouped<F, 0, 2048, false, false>);
     hipLaunchKernelGGL(kern, dim3(resident_blocks((const void*)kern, PF_GWPB * 64, lds)), block, lds, st, wq, ws, X,
@@ -1434,8 +1403,9 @@ void launch_grouped(const uint8_t* wq, const void* ws, const uint16_t* X, const 
   }
 }
 
-// gate_up then down for all experts of a grouped batch; with rmap, the gate_up token rows are
-// read from X (x_rows rows) through the slot -> row map instead of from a gathered xp
+// gate_up then down for all experts of a grouped batch; with rmap (and with packed weights always), the
+// gate_up token rows are read from X (x_rows rows, > 0 only then) through the slot -> row map instead of from a
+// gathered xp
 template <class F>
 int moe_prefill(const uint8_t* gu_q, const void* gu_s, const uint8_t* d_q, const void* d_s, const uint16_t* xp,
                 const int* offsets, const int* counts, uint16_t* act, float* y, int E, int H, int I, size_t gu_q_b,

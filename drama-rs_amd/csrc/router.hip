@@ -94,40 +94,38 @@ __global__ void __launch_bounds__(512)
     const int c = lane + WAVE * j;
     w[j] = c < KC ? ld16(W + (size_t)n * K + (size_t)c * 8) : make_uint4(0, 0, 0, 0);
   }
-  for (int m0 = 0; m0 < M; m0 += 4) {
-    uint4 av[4][NCH];
+  static_assert(GR_MAXM == 4, "all rows at once");
+  uint4 av[4][NCH];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + r < M ? m0 + r : M - 1;
+  for (int r = 0; r < 4; ++r) {
+    const int m = r < M ? r : M - 1;
 #pragma unroll
-      for (int j = 0; j < NCH; ++j) {
-        const int c = lane + WAVE * j;
-        av[r][j] = c < KC ? ld16(A + (size_t)m * K + (size_t)c * 8) : make_uint4(0, 0, 0, 0);
+    for (int j = 0; j < NCH; ++j) {
+      const int c = lane + WAVE * j;
+      av[r][j] = c < KC ? ld16(A + (size_t)m * K + (size_t)c * 8) : make_uint4(0, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      if (lane + WAVE * j < KC) {
+        const uint4 a = av[r][j], b = w[j];
+        acc = __builtin_fmaf(bf16_lo(b.x), bf16_lo(a.x), acc);
+        acc = __builtin_fmaf(bf16_hi(b.x), bf16_hi(a.x), acc);
+        acc = __builtin_fmaf(bf16_lo(b.y), bf16_lo(a.y), acc);
+        acc = __builtin_fmaf(bf16_hi(b.y), bf16_hi(a.y), acc);
+        acc = __builtin_fmaf(bf16_lo(b.z), bf16_lo(a.z), acc);
+        acc = __builtin_fmaf(bf16_hi(b.z), bf16_hi(a.z), acc);
+        acc = __builtin_fmaf(bf16_lo(b.w), bf16_lo(a.w), acc);
+        acc = __builtin_fmaf(bf16_hi(b.w), bf16_hi(a.w), acc);
       }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < NCH; ++j) {
-        if (lane + WAVE * j < KC) {
-          const uint4 a = av[r][j], b = w[j];
-          acc = __builtin_fmaf(bf16_lo(b.x), bf16_lo(a.x), acc);
-          acc = __builtin_fmaf(bf16_hi(b.x), bf16_hi(a.x), acc);
-          acc = __builtin_fmaf(bf16_lo(b.y), bf16_lo(a.y), acc);
-          acc = __builtin_fmaf(bf16_hi(b.y), bf16_hi(a.y), acc);
-          acc = __builtin_fmaf(bf16_lo(b.z), bf16_lo(a.z), acc);
-          acc = __builtin_fmaf(bf16_hi(b.z), bf16_hi(a.z), acc);
-          acc = __builtin_fmaf(bf16_lo(b.w), bf16_lo(a.w), acc);
-          acc = __builtin_fmaf(bf16_hi(b.w), bf16_hi(a.w), acc);
-        }
-      }
-      acc = wave_sum(acc);
-      const int m = m0 + r;
-      if (lane == 0 && m < M) {
-        float* c = C + (size_t)m * N + n;
-        *c = beta == 0.f ? acc : acc + beta * *c;
-      }
+    acc = wave_sum(acc);
+    if (lane == 0 && r < M) {
+      float* c = C + (size_t)r * N + n;
+      *c = beta == 0.f ? acc : acc + beta * *c;
     }
   }
 }
