@@ -1328,22 +1328,28 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// blocks of a kernel resident on the whole current device at once (occupancy x CUs), cached
-// per (kernel, device); launchers may be called from several host threads
+// blocks of a kernel resident on the whole current device at once (occupancy x CUs), kept
+// per kernel (36 of them: 9 per format) and device; launchers may be called from several host threads
 inline int resident_blocks(const void* kern, int threads, size_t lds) {
+  constexpr int KERNELS = 64, DEVICES = 16;
   static std::mutex mu;
-  static const void* keys[64];
-  static int devs[64], vals[64], n = 0;
+  static const void* keys[KERNELS];
+  static int vals[KERNELS][DEVICES], n = 0;  // 0: not asked for yet
   int dev = 0;
   (void)hipGetDevice(&dev);
   std::lock_guard<std::mutex> lock(mu);
-  for (int i = 0; i < n; ++i)
-    if (keys[i] == kern && devs[i] == dev) return vals[i];
+  int k = 0;
+  while (k < n && keys[k] != kern) ++k;
+  const bool keep = k < KERNELS && dev >= 0 && dev < DEVICES;
+  if (keep && k < n && vals[k][dev]) return vals[k][dev];
   int cus = 0, per = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, threads, lds);
   const int v = (per > 0 ? per : 1) * (cus > 0 ? cus : 256);
-  if (n < 64) keys[n] = kern, devs[n] = dev, vals[n] = v, ++n;
+  if (keep) {
+    if (k == n) keys[n++] = kern;
+    vals[k][dev] = v;
+  }
   return v;
 }
 
