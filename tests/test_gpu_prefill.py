@@ -720,3 +720,52 @@ def test_prefill_passes_few_tokens(kind, fmt, packed, counts):
     for p, q in ((a0.view(torch.bfloat16), a1.view(torch.bfloat16)), (y0, y1)):
         assert torch.equal(p.isnan(), q.isnan())
         assert torch.equal(p.nan_to_num(nan=0.0).view(p.dtype), q.nan_to_num(nan=0.0).view(p.dtype))
+
+
+@pytest.mark.parametrize("passes,packed", [(True, True), (True, False), (False, False)])
+def test_prefill_fp8_every_code(passes, packed):
+    """All 256 e4m3 codes in the expert weights of both grouped kernels: y against the float64 product of the
+    kernel's own act with the decoded weights, NaN exactly where a row of weights holds a NaN code."""
+    import torch
+
+    E, n, rows = 2, 40, 448
+    lib, P, st = D.lib(), D.ptr, D.stream_ptr()
+    g = torch.Generator(device="cuda").manual_seed(53)
+    L = {k: dev(v) for k, v in synth.make_layer(53, E=E, fmt="ref", kind="fp8", quick=True).items()
+         if k in ("gu_q", "gu_s", "d_q", "d_s")}
+    codes = torch.arange(256, dtype=torch.int64, device="cuda")
+    finite = codes[(codes & 127) != 127]
+    d = finite[torch.randint(0, 254, (E, H, I), generator=g, device="cuda")]
+    d[:, ::37, :256] = codes  # every code in some rows, two of them NaN
+    d[:, 5::37, :254] = finite
+    L["d_q"] = d.to(torch.uint8).contiguous()
+    W = dict(L)
+    if packed:
+        for q, nn, kk in (("gu_q", 2 * I, H), ("d_q", H, I)):
+            W[q] = torch.zeros_like(L[q])
+            lib.dr_moe_pack_fp8(P(L[q]), E, nn, kk, P(W[q]), st)
+    x = torch.randn(rows, H, generator=g, device="cuda").to(torch.bfloat16)
+    ros = torch.randint(0, rows, (n + 16,), generator=g, device="cuda", dtype=torch.int32)
+    cnt, off = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([n - 7, 7], [0, n - 7]))
+    act, y = torch.zeros(n, I, dtype=torch.bfloat16, device="cuda"), torch.zeros(n, H, device="cuda")
+    if passes:
+        getattr(lib, "dr_moe_prefill_rows" + ("_packed" if packed else "") + "_fp8")(
+            P(W["gu_q"]), P(W["gu_s"]), P(W["d_q"]), P(W["d_s"]), P(x), rows, P(ros), P(off), P(cnt), P(act), P(y), E, H,
+            I, st)
+    else:
+        xp = x[ros.long()].contiguous()
+        lib.dr_moe_prefill_fp8(P(L["gu_q"]), P(L["gu_s"]), P(L["d_q"]), P(L["d_s"]), P(xp), P(off), P(cnt), P(act), P(y),
+                               E, H, I, st)
+    torch.cuda.synchronize()
+    assert lib.dr_last_error() == 0 and act.isfinite().all() and act.any()
+    for e, sl in ((0, slice(0, n - 7)), (1, slice(n - 7, n))):
+        w = L["d_q"][e].view(torch.float8_e4m3fn).cpu().double()
+        s = L["d_s"][e].cpu().double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+        a, got = act[sl].cpu().double(), y[sl].cpu().double()
+        nan = w.isnan().any(1)
+        assert nan.sum() == len(range(0, H, 37))
+        assert got[:, nan].isnan().all() and got[:, ~nan].isfinite().all()
+        ws = (w * s)[~nan]
+        # 512 products, each sum in fp32: at most 512 roundings of 2^-24 of the sum of magnitudes
+        bound = 512 * 2.0 ** -24 * (a.abs() @ ws.abs().T)
+        assert ((got[:, ~nan] - a @ ws.T).abs() <= bound).all()
