@@ -280,8 +280,8 @@ void launch_gemm_mfma(const uint16_t* A, const uint16_t* W, float* C, int M, int
 }
 
 // The tile with the least cost a + b r, r the rounds of 256 tiles: fitted to the times of every tile over 5 to
-// 1024 rows, 33 to 16384 columns and K = 504 to 4096 (units of 10 ns at K = 2048, where the order is that of every
-// larger K, and at K = 512).  Few tiles: the smallest, whose waves have the fewest products; many: the large
+// 1024 rows, 33 to 16384 columns and K = 504 to 4096 (units of 10 ns at K = 512 and at K = 2048, where the order is that
+// of every larger K but for the 8-wave tile).  Few tiles: the smallest, whose waves have the fewest products; many: the large
 // ones, which load less per product, as long as their last round and their rows past M cost less than that saves.
 // us at K = 2048 for 16 x 16, 32 x 16 or 16 x 32, 32 x 32, 32 x 16 tiles of 8 waves: 100 x 257 5.8 / 8.1 / 12.0 / 8.7,
 // 300 x 257 9.4 / 8.1 / 12.2 / 8.8, 512 x 257 13.0 / 14.6 / 12.2 / 14.3, 1024 x 257 20.0 / 21 / 23.5 / 19.9, 5 x 4104 7.3 /
@@ -300,7 +300,12 @@ void launch_gemm(const uint16_t* A, const uint16_t* W, float* C, int M, int N, i
   };
   const long long c11 = cost(m16 * n16, 240, 120, 230, 350), c21 = cost(m32 * n16, 200, 175, 150, 655);
   const long long c12 = cost(m16 * n32, 200, 176, 150, 660), c22 = cost(m32 * n32, 100, 390, 90, 1120);
-  const long long c8 = cost(m32 * n16, 220, 164, 330, 550);
+  // 8 waves: K = 4096 runs with chunk bounds (above) and costs more (700 x 2048 130 us against 123 for 32 x 32).  K = 2048 at three rounds: 1024 x 257 takes 19.8 us
+  // like 16 x 16 tiles (20.0), but beside other kernels, which the 16-wave blocks of those leave no room, less: a
+  // prefill layer of 1024 rows with its shared expert on a second stream 237 us against 250
+  const long long c8 = K == 4096   ? cost(m32 * n16, 220, 164, 200, 630)
+                       : K == 2048 ? cost(m32 * n16, 220, 164, 315, 550)
+                                   : cost(m32 * n16, 220, 164, 345, 550);
   const long long c = std::min({c11, c21, c12, c22, c8});
   if (c == c11) launch_gemm_mfma<NCH, 1, 1, 16>(A, W, C, M, N, K, beta, st);
   else if (c == c21) launch_gemm_mfma<NCH, 2, 1, 16>(A, W, C, M, N, K, beta, st);
