@@ -1359,12 +1359,13 @@ inline int resident_blocks(const void* kern, int threads, size_t lds) {
 // reference layout).  Whole prefill layers at 256 experts, k_grouped ->
 // k_grouped_pass: int4 300 rows 147 -> 150 us, 449 rows 173 -> 174, 512 (reference layout) 201 -> 194, 1024
 // 303 -> 264, hot experts 460 / 900 rows 170 / 249 -> 160 / 223; fp8 12 rows 94 -> 104, 300 rows 203 -> 207,
-// 460 rows 226 -> 227, 600 rows 258 -> 243.  Fewer experts, gate_up and down alone, time over k_grouped's at the 14
-// picks: int4 144 / 112 / 96 / 72 / 48 / 24 experts 1.12 / 1.08 / 1.18 / 1.34 / 1.67 / 2.3 (hot experts still 1.09 at 352
-// rows of 128), fp8 1.06 / 0.98 / 1.00 / 1.20 / 1.39 / 1.96, its copy 1.07 / 1.01 / 1.01 / 1.22 / 1.20 / 1.69; from the rows
-// above on 0.75 to 1.05 (int4) and 0.50 to 1.05 (fp8).  The number of rows is only known where they come through
-// a row map; elsewhere (x_rows 0) k_grouped stays.  The number of picks is not known at all: at 2 picks per row
-// the kernel chosen from 448 rows and 256 experts on takes 3 to 11% longer than k_grouped would.
+// 460 rows 226 -> 227, 600 rows 258 -> 243.  Fewer experts, gate_up and down alone over changing weights, time over
+// k_grouped's from 14 picks on, uniform / hot routings: below those rows int4 0.80 to 2.2 / 0.83 to 2.4, fp8 0.66 to 2.1 / 0.74
+// to 2.2, its copy 0.70 to 1.7 / 0.78 to 1.8 (the low ends 64 experts from 20 picks on, whose items are one whole round of
+// the chip, and 300 picks and more); from them on int4 0.78 to 1.02 / 0.74 to 1.11, fp8 0.53 to 1.05 / 0.52 to 1.13, its copy
+// 0.59 to 1.03 / 0.58 to 1.04.  The number of rows is only known where they come through a row map; elsewhere (x_rows 0)
+// k_grouped stays.  The number of picks is not known at all: at 2 picks per row the kernel chosen from 448 rows and 256
+// experts on takes 3 to 14% longer than k_grouped would.
 template <class F>
 inline bool use_passes(int x_rows, int E, bool packed) {
   return x_rows >= (F::paired ? 448 : packed ? 384 : 256) && (long long)x_rows * 8 >= 14ll * E;

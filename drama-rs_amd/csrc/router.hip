@@ -300,9 +300,10 @@ void launch_gemm(const uint16_t* A, const uint16_t* W, float* C, int M, int N, i
   };
   const long long c11 = cost(m16 * n16, 240, 120, 230, 350), c21 = cost(m32 * n16, 200, 175, 150, 655);
   const long long c12 = cost(m16 * n32, 200, 176, 150, 660), c22 = cost(m32 * n32, 100, 390, 90, 1120);
-  // 8 waves: K = 4096 runs with chunk bounds (above) and costs more (700 x 2048 130 us against 123 for 32 x 32).  K = 2048 at three rounds: 1024 x 257 takes 19.8 us
-  // like 16 x 16 tiles (20.0), but beside other kernels, which the 16-wave blocks of those leave no room, less: a
-  // prefill layer of 1024 rows with its shared expert on a second stream 237 us against 250
+  // 8 waves: K = 4096 runs with chunk bounds (above) and costs more (700 x 2048 130 us against 123 for 32 x 32).
+  // K = 2048 at three rounds: 1024 x 257 takes 19.8 us, level with 16 x 16 tiles (20.0), but beside other kernels, which
+  // the 16-wave blocks of those leave no room, it is the shorter one: a prefill layer of 1024 rows with its shared
+  // expert on a second stream 237 us against 250
   const long long c8 = K == 4096   ? cost(m32 * n16, 220, 164, 200, 630)
                        : K == 2048 ? cost(m32 * n16, 220, 164, 315, 550)
                                    : cost(m32 * n16, 220, 164, 345, 550);
