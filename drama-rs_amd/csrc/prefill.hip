@@ -636,7 +636,9 @@ __global__ void __launch_bounds__(PF_GWPB * 64)
 // pair per group.  An output's sums depend neither on the pass or tile its token falls in nor on the
 // kernel (the same operations in the same order as k_grouped, so the same bits).
 // What bounds it: at one token tile per pass the steps run at the HBM rate (1.55 us for 36.8 KB per
-// CU, 6.1 TB/s); with two int4 tiles the dequantisation and MFMA issue of a step (1.9 us) do.
+// CU, 6.1 TB/s); with two int4 tiles the dequantisation and MFMA issue of a step (1.9 us: at 1024 rows the vector units
+// issue in 56% of the clocks, the matrix units are busy in 22%), and second passes read their weights again (1.56x
+// the weight bytes at 1024 rows).
 // Measured (tile-step copy, gate_up / down, k_grouped -> k_grouped_pass): int4 1024 rows 143 / 78 -> 112 / 66 us,
 // fp8 600 rows with hot experts 124 / 68 -> 117 / 60 us; int4 300 rows 68 / 37.7 -> 67 / 41 us (use_passes).
 // Not kept: 16-row tiles with two blocks per CU (132 / 72 us at 1024 rows), passes of 48 and 64

@@ -289,7 +289,9 @@ int dr_moe_shared_prefill_bf16s(const int8_t* sgu_q, const dr_bf16* sgu_s, const
 
 /* Small decode batches (a few tokens decoded together, e.g. benchmark configuration 5's
  * batch 4): the batch-1 chain dr_router_topk -> dr_moe_decode(_fp8) for `rows` independent
- * rows in three launches instead of a prefill-style grouping.  Row r uses x + r k (f32),
+ * rows instead of a prefill-style grouping: a router launch per 8 rows, then int4 one gate_up
+ * launch for the rows in whole fours, a second for the one to three left, and one down
+ * launch; FP8 a gate_up and a down launch per four rows.  Row r uses x + r k (f32),
  * logits + r (e + 1), idx/wts + r topk, sgate + r; the experts of each row are streamed once
  * per row and the shared expert once for up to four rows.  Routing of each row is bit-exact
  * with dr_router_topk on that row.  No reference counterpart (the engine decodes one token
