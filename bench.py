@@ -468,7 +468,7 @@ def main():
             import oracle as O
 
             # every core this process may use: the affinity set, bounded by OMP_NUM_THREADS
-            # where the host sets it (one GPU's share of the GPU box's host is 16 cores)
+            # where the host sets it (one card's share of its host is 16 cores)
             avail = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else (os.cpu_count() or 1)
             threads = min(avail, int(os.environ.get("OMP_NUM_THREADS", avail)))
             hl0 = dict(hl, router=h["router"].view(np.uint16), nw=h["nw"])
